@@ -150,6 +150,14 @@ __device__ __forceinline__ void lds_dma16(const void *base, uint32_t off, void *
         : "v"(off), "s"(sb), "s"(lds));
 }
 
+// The lane's index in its wave, formed where it is used (two instructions) so
+// that no register holds it, or anything derived from it, across a tile loop.
+__device__ __forceinline__ int fresh_lane() {
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+}
+
 // s * v for s, v < 2^24 with the product below 2^32 (v_mul_u32_u24, a
 // full-rate instruction; s wave-uniform).  Written as assembly: from the
 // same product in C the compiler forms v_mad_u64_u32, a quarter-rate

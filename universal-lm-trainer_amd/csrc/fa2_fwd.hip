@@ -188,8 +188,7 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
     // an opaque move so that nothing derived from it stays live across the
     // loop).  Recomputing every tile cost ~25 VALU instructions per tile.
     auto tile_offsets = [&](int k0, uint32_t(&ko)[2], uint32_t(&vo)[2]) FA2_INLINE {
-        int ln = lane;
-        if (NARROW) asm volatile("v_mov_b32 %0, %1" : "=v"(ln) : "v"(lane));
+        const int ln = NARROW ? fresh_lane() : lane;
         const int lrow = ln >> 3;
         const int kch[2] = {(ln & 7) ^ swz_rows(lrow), (ln & 7) ^ swz_rows(lrow + 8)};
         const int vch = (ln & 7) ^ swz_tr(lrow);
@@ -230,14 +229,13 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
         } else if (NARROW) {
             // An opaque slot address: the read stays in the loop instead of
             // being hoisted into four live registers.  With keep-bit words
-            // it is formed from an opaque copy of the lane index every tile,
-            // so that no register holds it across the loop (kept live, that
-            // variant spilled it to scratch and reloaded it at every tile).
+            // it is formed from a fresh lane index every tile, so that no
+            // register holds it across the loop (kept live, that variant
+            // spilled it to scratch and reloaded it at every tile, and a
+            // scratch load's wait also drains the tile transfers in flight).
             uint32_t oa;
             if (DMASK) {
-                uint32_t ln;
-                asm volatile("v_mov_b32 %0, %1" : "=v"(ln) : "v"(lane));
-                oa = lds_addr(&sOff[64 * wave]) + 16u * ln;
+                oa = lds_addr(&sOff[64 * wave]) + 16u * (uint32_t)fresh_lane();
             } else {
                 oa = lds_addr(&sOff[64 * wave]) + 16u * (uint32_t)lane;
                 asm volatile("" : "+v"(oa));
@@ -556,14 +554,13 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
             float rs;
-            if (!DMASK && t == 0) {
+            if (t == 0) {
                 // First tile: msc is -inf, so P against it would only fail
                 // the overflow check into the cold path (a second P pass).
                 // Take the row max from the live scores directly, as the
                 // cold path would (with O and l still zero its rescale is a
                 // no-op), so the result is the same bits; -inf when every key
-                // is masked.  (With keep-bit words this copy would spill;
-                // they keep the cold path, with the same result.)
+                // is masked.
                 float mx = s[qb][0][0];
 #pragma unroll
                 for (int kb = 0; kb < 2; ++kb)
@@ -635,16 +632,23 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
         // Unrolled over the NSK stages (tile t sits in stage t % NSK, and
         // every wave starts at tile 0), so that each copy's stage is a
         // constant and the operand reads address LDS through instruction
-        // offsets, with no per-tile address arithmetic.  (With keep-bit
-        // words the copies would spill: one copy, the stage at run time.)
-        constexpr int U = DMASK ? 1 : NSK;
-        for (int t0 = 0; t0 < ntiles; t0 += U) {
+        // offsets, with no per-tile address arithmetic.
+        // DMASK: the word of (tile t, half 0, query qw0) as a running scalar
+        // address and the tile's run length; a lane adds its row and half as
+        // a 32-bit offset.  (dmask_word per tile and lane took four 64-bit
+        // vector multiply-adds and a scratch reload whose wait drained the
+        // next tile's transfers; without either, and with the loop unrolled
+        // as below, the forward with words goes from 238 to 223.5 us at B=15
+        // H=12 S=2050 and from 139.6 to 135 at B=32 S=1024.)
+        uint64_t dm = DMASK ? (uint64_t)(uintptr_t)(a.drop_mask + dmask_word(CAUSAL, bh, S, 0, 0, qw0)) : 0u;
+        int dn = DMASK ? dmask_run(CAUSAL, S, 0) : 0;
+        for (int t0 = 0; t0 < ntiles; t0 += NSK) {
 #pragma unroll
-            for (int ph = 0; ph < U; ++ph) {
+            for (int ph = 0; ph < NSK; ++ph) {
                 const int t = t0 + ph;
                 if (t >= ntiles) break;
                 uint32_t w = 0;
-                if (t <= tlast) w = inorder_tile(t, U == 1 ? stage_of(t) : ph, s, p);
+                if (t <= tlast) w = inorder_tile(t, ph, s, p);
                 if (t + 1 < ntiles) {
                     if (DMASK && FA2_FWD_STORE_SLACK && t >= 1 && t - 1 <= tlast)
                         wait_tiles_st(min(NSK - 2, ntiles - 2 - t));
@@ -653,9 +657,16 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
                     lds_barrier();
                     if (t + NSK < ntiles) issue_next();
                 }
-                if (DMASK && t <= tlast) {
-                    const int q = qw0 + c;   // QB == 1
-                    if (q < S) a.drop_mask[dmask_word(CAUSAL, bh, S, kbase / KT + t, g2, q)] = w;
+                if (DMASK) {
+                    if (t <= tlast) {
+                        const int ln = fresh_lane(), r = ln & 31;   // query qw0 + r (QB == 1)
+                        if (qw0 + r < S)
+                            *reinterpret_cast<uint32_t *>(dm + 4u * (mul_u24((uint32_t)dn, (uint32_t)ln >> 5) + (uint32_t)r)) = w;
+                    }
+                    // Next tile's run; a 128-key block's runs start 128 queries later.
+                    const bool next_block = CAUSAL && (t & 1);
+                    dm += 4 * (int64_t)(2 * dn - (next_block ? 128 : 0));
+                    dn -= next_block ? 128 : 0;
                 }
             }
         }
