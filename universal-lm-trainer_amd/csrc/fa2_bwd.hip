@@ -142,7 +142,7 @@ __global__ __launch_bounds__(256, NARROW ? DQ_NARROW_WAVES : 2) void bwd_dq_pipe
     _Float16 *dQp = a.dq + b * a.dqsb + h * a.dqsh;
     float *Dp = a.delta + (int64_t)bh * S;
 
-    const int q_wg0 = qblk * QWG;
+    const int q_wg0 = query_block_base(CAUSAL, S, QWG) + qblk * QWG;   // below 0 only in a partial block 0
     const int qw0 = q_wg0 + wave * 32 * QB;
     const float scale2 = a.scale2;
 
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256, NARROW ? DQ_NARROW_WAVES : 2) void bwd_dq_pipe
     const int ntiles = (kend + DQ_KT - 1) / DQ_KT;
     // Last key tile of this wave (-1: none).  The wave's first query is a
     // multiple of the tile size, so only that tile can need a mask.
-    const int tlast = (qw0 >= S) ? -1 : CAUSAL ? (min(qw0 + 32 * QB, S) - 1) / DQ_KT : ntiles - 1;
+    const int tlast = (qw0 >= S || qw0 < 0) ? -1 : CAUSAL ? (min(qw0 + 32 * QB, S) - 1) / DQ_KT : ntiles - 1;
 
     // Stage of tile t (t >= 0; unsigned, so a power-of-two count is a mask).
     auto stage_of = [](int t) FA2_INLINE { return (int)((uint32_t)t % (uint32_t)NSK); };
@@ -190,7 +190,8 @@ __global__ __launch_bounds__(256, NARROW ? DQ_NARROW_WAVES : 2) void bwd_dq_pipe
     uint32_t stn = 0;    // its stage
     const uint32_t lds_kv = lds_addr(&sKV[0][0][0]) + 2048u * (uint32_t)wave;
     // DMASK: the wave's 64 (NARROW: 32) words per half g2 of each tile (rows
-    // past S are within the mask's padded rows), 4 bytes per lane.
+    // past S are within the mask's padded rows; a wave below query 0 moves
+    // words of the first queries and uses none), 4 bytes per lane.
     const uint32_t lds_mq = lds_addr(&sMQ[0][wave][0][0]);
     {
         // (With S < DQ_KT every tile is partial and recomputes its offsets,
@@ -223,7 +224,7 @@ __global__ __launch_bounds__(256, NARROW ? DQ_NARROW_WAVES : 2) void bwd_dq_pipe
         if (DMASK) {
 #pragma unroll
             for (int half = 0; half < 2; ++half)
-                lds_dma4_at((uint64_t)(uintptr_t)(a.drop_mask + dmask_word(CAUSAL, bh, S, kn / DQ_KT, half, qw0)),
+                lds_dma4_at((uint64_t)(uintptr_t)(a.drop_mask + dmask_word(CAUSAL, bh, S, kn / DQ_KT, half, max(qw0, 0))),
                             4u * (uint32_t)(NARROW ? (lane & 31) : lane),   // NARROW: 32 words, lanes 32.. repeat
                             lds_mq + stn * (uint32_t)sizeof(sMQ[0]) + 256u * (uint32_t)half);
         }
@@ -237,14 +238,15 @@ __global__ __launch_bounds__(256, NARROW ? DQ_NARROW_WAVES : 2) void bwd_dq_pipe
         if (t < ntiles) issue_next();
 
     // Resident Q^T / dO^T operands, delta and log2-scaled LSE of the wave's
-    // queries (rows past S: row S - 1 and LSE = +inf, so P = dS = 0).
+    // queries (rows past S: row S - 1, rows below 0: row 0, and LSE = +inf,
+    // so P = dS = 0).
     h8 qf[QB][4], dof[QB][4];
     float lse2[QB], dl[QB];
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
         const int q = qw0 + 32 * qb + c;
-        const bool valid = q < S;
-        const int qr = min(q, S - 1);
+        const bool valid = q >= 0 && q < S;
+        const int qr = max(min(q, S - 1), 0);
         float part = 0.f;
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
@@ -480,6 +482,7 @@ __global__ __launch_bounds__(256, NARROW ? DQ_NARROW_WAVES : 2) void bwd_dq_pipe
     // first, waves 2, 3 the second.
     static_assert(NARROW ? sizeof(sKV) >= DQ_NW * 4096 : (NSK == 4 && QB == 2 && sizeof(sKV[0]) == 16384),
                   "dQ staging layout");
+    if (qw0 < 0) return;   // (past the last barrier)
     const float sc = a.scale;
     const bool dq16 = ((a.dqsb | a.dqsh | a.dqss) & 7) == 0;
     char *const stg = NARROW ? reinterpret_cast<char *>(&sKV[0][0][0]) + 4096 * wave

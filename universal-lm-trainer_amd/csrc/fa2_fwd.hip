@@ -142,7 +142,7 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
     _Float16 *Op = a.o + b * a.osb + h * a.osh;
     float *Lp = a.lse + b * a.lsb + h * a.lsh;
 
-    const int q_wg0 = qblk * QWG;
+    const int q_wg0 = query_block_base(CAUSAL && !SPLIT, S, QWG) + qblk * QWG;   // below 0 only in a partial block 0
     const int qw0 = q_wg0 + wave * 32 * QB;   // this wave's queries: qw0 .. qw0 + 32*QB - 1
     const float scale2 = a.scale2;
 
@@ -154,19 +154,19 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
     // Last key tile this wave computes (-1: none).  Every wave still joins
     // every barrier and moves its share of every tile.
     const int kw_end = min(CAUSAL ? min(qw0 + 32 * QB + coff, Sk) : Sk, kend);   // keys the wave's queries reach
-    const int tlast = (qw0 >= S || kw_end <= kbase) ? -1 : (kw_end - 1 - kbase) / KT;
+    const int tlast = (qw0 >= S || qw0 < 0 || kw_end <= kbase) ? -1 : (kw_end - 1 - kbase) / KT;
     // Tiles before tsteady are visible to every query of the wave (the
     // steady, mask-free path); the rest run the general path.
     const int tsteady = CAUSAL ? min(tlast, max(qw0 + coff + 1 - kbase, 0) / KT) : tlast;
 
     // Q^T operand of d-step st: lane holds Q[q][16*st + 8*g2 + e].  Rows past
-    // S load row S - 1 (unconditional loads stay in flight together); those
-    // lanes' results are never stored.  Loaded before the first tiles, so
+    // S load row S - 1 and rows below 0 row 0 (unconditional loads stay in
+    // flight together); those lanes' results are never stored.  Loaded before the first tiles, so
     // waiting for a tile also covers them.
     h8 qf[QB][4];
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
-        const _Float16 *qrow = Qp + (int64_t)min(qw0 + 32 * qb + c, S - 1) * a.qss + 8 * g2;
+        const _Float16 *qrow = Qp + (int64_t)max(min(qw0 + 32 * qb + c, S - 1), 0) * a.qss + 8 * g2;
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
             const h8 v = *reinterpret_cast<const h8 *>(qrow + 16 * st);
@@ -847,6 +847,7 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
         }
         return;
     }
+    if (qw0 < 0) return;   // (past the last barrier)
     // Epilogue: O = acc / l (l == 0 -> 0), LSE = (m*scale2 + log2 l) * ln 2.
     // O rows leave through this wave's 4 KB slice of the stages.
     const bool o16 = ((a.osb | a.osh | a.oss) & 7) == 0;
