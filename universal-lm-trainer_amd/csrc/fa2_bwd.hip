@@ -142,7 +142,7 @@ __global__ __launch_bounds__(256, NARROW ? DQ_NARROW_WAVES : 2) void bwd_dq_pipe
     _Float16 *dQp = a.dq + b * a.dqsb + h * a.dqsh;
     float *Dp = a.delta + (int64_t)bh * S;
 
-    const int q_wg0 = query_block_base(CAUSAL, S, QWG) + qblk * QWG;   // below 0 only in a partial block 0
+    const int q_wg0 = a.qbase + qblk * QWG;   // below 0 only in a partial block 0
     const int qw0 = q_wg0 + wave * 32 * QB;
     const float scale2 = a.scale2;
 
@@ -1000,6 +1000,7 @@ static void launch_dq_t(const BwdArgs &a_in, bool causal, bool dropout, hipStrea
     a.hgroup = (a.B * a.H) % 8 == 0 && a.S <= FA2_DQ_GROUP_MAX_S ? 16 : 0;
     const int qwg = NARROW && !(dropout && a.drop_mask != nullptr) ? DQ_NW * 32 : DQ_QWG;
     const dim3 grid((unsigned)((a.S + qwg - 1) / qwg * a.B * a.H)), block(256);
+    a.qbase = query_block_base(causal, a.S, qwg, grid.x, (int64_t)(qwg == DQ_QWG ? 2 : DQ_NARROW_WAVES) * device_cus());
     const bool dmask = dropout && a.drop_mask != nullptr;
     if (causal) {
         if (dmask)

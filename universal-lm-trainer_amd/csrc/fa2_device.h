@@ -435,22 +435,6 @@ __device__ __forceinline__ int64_t dmask_word(bool causal, int bh, int S, int t6
     return (int64_t)bh * head + before + (int64_t)(t64 & 1) * 2 * n + (int64_t)g2 * n + (q - 128 * j);
 }
 
-// First query of the head's query block 0 (blocks of `qwg` queries).  Under
-// the causal mask the blocks are moved down by whole 64-query groups until the
-// last one ends within 64 queries of S: a partial block is then block 0, which
-// reaches the fewest keys, where with blocks counted from query 0 it is the
-// last, whose few queries run the head's whole key range.  Waves whose queries
-// lie below 0 (block 0 only; all of a wave's or none, waves hold 32 or 64)
-// compute and store nothing.  Whole groups keep every wave on the tile grid:
-// ending the last block exactly at S gave each two-block dQ wave one more
-// masked tile (4-5% slower at S = 1500 and 1985).  Measured against blocks
-// counted from 0 (H = 12, about 24k rows): forward 72.2 -> 67.6 us at
-// S = 1030, dQ pass 100.5 -> 92.3 us there and, with keep words, 87.2 -> 75.4
-// at S = 632; equal where the last block is nearly full (505, 760, 1500, 1985).
-__device__ __forceinline__ int query_block_base(bool causal, int S, int qwg) {
-    return causal ? -(((S + qwg - 1) / qwg * qwg - S) & ~63) : 0;
-}
-
 // Workgroup order of the query-block kernels (forward, dQ pass): workgroup L
 // of a grid of nq * BH -> its query slot (0 = the head's last, heaviest
 // query block) and its head bh.  Workgroups go to the 8 XCDs in turn

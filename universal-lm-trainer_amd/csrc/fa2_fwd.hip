@@ -142,7 +142,7 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
     _Float16 *Op = a.o + b * a.osb + h * a.osh;
     float *Lp = a.lse + b * a.lsb + h * a.lsh;
 
-    const int q_wg0 = query_block_base(CAUSAL && !SPLIT, S, QWG) + qblk * QWG;   // below 0 only in a partial block 0
+    const int q_wg0 = a.qbase + qblk * QWG;   // below 0 only in a partial block 0
     const int qw0 = q_wg0 + wave * 32 * QB;   // this wave's queries: qw0 .. qw0 + 32*QB - 1
     const float scale2 = a.scale2;
 
@@ -1072,6 +1072,7 @@ template <bool SPLIT>
 void launch_fwd_t(const FwdArgs &a_in, bool causal, bool dropout, hipStream_t st) {
     FwdArgs a = a_in;
     a.hgroup = 0;
+    a.qbase = 0;
     const dim3 block(NW * 64);
     // Keep-bit words only from the unsplit forward (the training path).
     const bool dmask = !SPLIT && dropout && a.drop_mask != nullptr;
@@ -1085,6 +1086,7 @@ void launch_fwd_t(const FwdArgs &a_in, bool causal, bool dropout, hipStream_t st
     const int64_t narrow_wgs = (int64_t)((a.S + qwg_of(1) - 1) / qwg_of(1)) * a.B * a.H;
     if (!SPLIT && FA2_FWD_NARROW && narrow_wgs >= (int64_t)NARROW_WAVES * device_cus()) {
         if ((a.B * a.H) % 8 == 0 && a.S <= FA2_FWD_GROUP_MAX_S) a.hgroup = 16;
+        a.qbase = query_block_base(causal, a.S, qwg_of(1), narrow_wgs, (int64_t)NARROW_WAVES * device_cus());
         if (causal) {
             if (dmask) launch_narrow<true, true, true>(a, st);
             else if (dropout) launch_narrow<true, true, false>(a, st);
@@ -1106,6 +1108,8 @@ void launch_fwd_t(const FwdArgs &a_in, bool causal, bool dropout, hipStream_t st
                      (int64_t)((a.S + qwg_of(2) - 1) / qwg_of(2)) * a.B * a.H >= 2 * (int64_t)device_cus();
     const int nqblk = (a.S + (two ? qwg_of(2) : qwg_of(1)) - 1) / (two ? qwg_of(2) : qwg_of(1));
     const dim3 grid((unsigned)(nqblk * a.B * a.H * (SPLIT ? a.nsplit : 1)));
+    if (!SPLIT)
+        a.qbase = query_block_base(causal, a.S, two ? qwg_of(2) : qwg_of(1), grid.x, 2 * (int64_t)device_cus());
     if (causal) {
         if (two) {
             if (dropout)

@@ -33,6 +33,7 @@ struct FwdArgs {
     uint32_t *drop_mask;
     // Workgroup order (query_block_order): heads per group, 0 = plain order.
     int hgroup;
+    int qbase;           // first query of query block 0 (query_block_base)
 };
 
 struct BwdArgs {
@@ -64,6 +65,7 @@ struct BwdArgs {
     bool dkv_pair;
     // dQ pass workgroup order (query_block_order): heads per group, 0 = plain.
     int hgroup;
+    int qbase;           // dQ pass: first query of query block 0 (query_block_base)
 };
 
 struct RopeArgs {
@@ -77,6 +79,26 @@ struct RopeArgs {
     // aligned: the vector kernel; otherwise the 4-byte one.
     bool vec16;
 };
+
+// First query of a head's query block 0 in the forward and the dQ pass
+// (blocks of `qwg` queries, `wgs` workgroups in all, `slots` of them resident).
+// Under the causal mask the blocks are moved down by whole 64-query groups until
+// the last one ends within 64 queries of S: a partial block is then block 0,
+// which reaches the fewest keys, where with blocks counted from query 0 it is
+// the last, whose few queries run the head's whole key range.  Waves whose
+// queries lie below 0 (block 0 only; all of a wave's or none, waves hold 32 or
+// 64) compute and store nothing.  Whole groups keep every wave on the tile
+// grid: ending the last block exactly at S gave each two-block dQ wave one more
+// masked tile (4-5% slower at S = 1500 and 1985).  Measured against blocks
+// counted from 0 (H = 12, about 24k rows): forward 72.2 -> 67.6 us at
+// S = 1030, dQ pass 100.5 -> 92.3 us there and, with keep words, 87.2 -> 75.4
+// at S = 632; equal where the last block is nearly full (505, 760, 1500, 1985).
+// A grid that is resident at once keeps the blocks at 0: there the longest
+// workgroup sets the time, and one with fewer active waves is shorter (forward
+// of 64 heads at S = 700 13.5 us, moved 14.2).
+inline int query_block_base(bool causal, int S, int qwg, int64_t wgs, int64_t slots) {
+    return causal && wgs > slots ? -(((S + qwg - 1) / qwg * qwg - S) & ~63) : 0;
+}
 
 // Compute units of the current device (cached per device; 256 on MI355X).
 // Launchers use it to size grids against the slots of two workgroups per CU.
