@@ -1,0 +1,62 @@
+"""Decode (one query, no dropout): cache lengths around the kernel's 64-key blocks, its eight waves'
+512-key strides and the binding's slice rule, with plain and with streaming loads, and the merge of
+more than 64 slices."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+# O is rounded to fp16 (2^-11 of values up to ~4 on N(0,1) inputs with few keys) and the scores are fp32.
+O_TOL = 2e-3
+
+
+def reference(q, k, v, keys):
+    s = torch.matmul(q.float(), k[:, :, :keys].float().transpose(-1, -2).contiguous()) * 0.125
+    return torch.matmul(torch.softmax(s, dim=-1), v[:, :, :keys].float()), torch.logsumexp(s, dim=-1)
+
+
+@pytest.mark.parametrize("B,H,Sk", [(1, 3, 1), (1, 3, 63), (2, 3, 65), (1, 12, 512), (1, 12, 513), (1, 12, 1535),
+                                    (1, 12, 1537), (2, 65, 1600), (8, 12, 3413), (8, 12, 3414), (3, 100, 1001)])
+@pytest.mark.parametrize("hidden", [0, 1])
+def test_decode_lengths(fa, B, H, Sk, hidden):
+    """(8, 12, 3413) is the longest cache of at most 80 MiB and takes plain loads, (8, 12, 3414) streams.
+    hidden: keys past the query's causal limit, in a cache that is a view of a longer one."""
+    print(f"case decode B={B} H={H} Sk={Sk} hidden={hidden}", flush=True)
+    g = torch.Generator().manual_seed(Sk + H)
+    q = torch.randn(B, H, 1, 64, generator=g).half().to(DEV)
+    k, v = (torch.randn(B, H, Sk + 7, 64, generator=g).half().to(DEV)[:, :, :Sk] for _ in range(2))
+    keys = max(1, Sk - hidden)
+    o, lse = fa.extension().fa_fwd_kv(q, k, v, True, 0.125, keys - 1, 0)
+    ro, rl = reference(q, k, v, keys)
+    assert (o.float() - ro).abs().max().item() <= O_TOL
+    assert (lse - rl).abs().max().item() <= 1e-3
+
+
+@pytest.mark.parametrize("nsplit", [5, 64, 65, 200])
+def test_decode_many_slices(fa, nsplit):
+    """The merge reads slices 64 at a time; slices past the cache's 157 blocks are empty."""
+    print(f"case decode slices {nsplit}", flush=True)
+    g = torch.Generator().manual_seed(nsplit)
+    q = torch.randn(1, 2, 1, 64, generator=g).half().to(DEV)
+    k, v = (torch.randn(1, 2, 10001, 64, generator=g).half().to(DEV) for _ in range(2))
+    o, lse = fa.extension().fa_fwd_kv(q, k, v, True, 0.125, 10000, nsplit)
+    ro, rl = reference(q, k, v, 10001)
+    assert (o.float() - ro).abs().max().item() <= O_TOL
+    assert (lse - rl).abs().max().item() <= 1e-3
+
+
+def test_decode_merge_edges(fa):
+    """The merge of slices gives NaN where a slice's softmax met an infinite score (inf - inf), and a
+    query that sees no key gives O = 0 and LSE = -inf with one slice and with several."""
+    print("case decode merge edges", flush=True)
+    ext = fa.extension()
+    q = torch.ones(1, 1, 1, 64, device=DEV).half()
+    k = torch.zeros(1, 1, 2000, 64, device=DEV).half()
+    v = torch.ones_like(k)
+    k[0, 0, 700, 3] = float("inf")
+    o, _ = ext.fa_fwd_kv(q, k, v, True, 0.125, 1999, 4)
+    assert torch.isnan(o).all()
+    for nsplit in (1, 4):
+        o, lse = ext.fa_fwd_kv(q, k, v, True, 0.125, -1, nsplit)
+        assert (o == 0).all() and (lse == float("-inf")).all(), nsplit

@@ -47,6 +47,8 @@
 #include "fa2_device.h"
 #include "fa2_kernels.h"
 
+#include <algorithm>
+
 namespace fa2 {
 namespace {
 
@@ -866,30 +868,55 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
 // Merges the slices of a split forward: with M the largest reference max of
 // a query's slices and w_s = 2^(m_s - M), O = sum_s w_s O_s / sum_s w_s l_s
 // and LSE = (M + log2 sum_s w_s l_s) ln 2 (a query no slice saw: O = 0,
-// LSE = -inf).  16 threads per query, 4 of its 64 columns each.
+// LSE = -inf).  G groups of 16 lanes per query: each lane reads one slice's
+// max and sum (16 G slices at a time), then group g takes slices g, g + G, ...,
+// 4 of the 64 columns per lane, so that no load waits for another slice's.
+// Latency bound (3.8 us for a few rows, launch included): G = 4 from five
+// slices on (16 slices of 12 rows 6.1 -> 3.9 us, 8 slices of 3072 rows
+// 5.9 -> 4.1), G = 1 for fewer, where the rows alone fill the card.
+template <int G>
 __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdArgs a) {
-    const int S = a.S;
+    constexpr int LPR = 16 * G;   // lanes per query
+    const int S = a.S, nsplit = a.nsplit;
     const int64_t BHS = (int64_t)a.B * a.H * S;
-    const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);   // (b*H + h)*S + q
-    if (row >= BHS) return;
-    const int part = threadIdx.x & 15;
+    const int64_t row = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;   // (b*H + h)*S + q
+    if (row >= BHS) return;   // whole groups leave together; shuffles stay inside them
+    const int lane = threadIdx.x % LPR, part = lane & 15, grp = lane >> 4;
     const int bh = (int)(row / S), q = (int)(row - (int64_t)bh * S);
     const int b = bh / a.H, h = bh - b * a.H;
-    float M = -INFINITY;
-    for (int s = 0; s < a.nsplit; ++s) M = fmaxf(M, a.part_ml[2 * (s * BHS + row)]);
+    auto slice_ml = [&](int s) FA2_INLINE {
+        return s < nsplit ? *reinterpret_cast<const f2 *>(a.part_ml + 2 * (s * BHS + row)) : f2{-INFINITY, 0.f};
+    };
+    const f2 ml0 = slice_ml(lane);
+    float M = ml0[0];
+    for (int s0 = LPR; s0 < nsplit; s0 += LPR) M = fmaxf(M, slice_ml(s0 + lane)[0]);
+#pragma unroll
+    for (int off = 1; off < LPR; off <<= 1) M = fmaxf(M, __shfl_xor(M, off));
     float lsum = 0.f;
     f4 acc = {0.f, 0.f, 0.f, 0.f};
     if (M != -INFINITY) {
-        for (int s = 0; s < a.nsplit; ++s) {
-            const f2 ml = *reinterpret_cast<const f2 *>(a.part_ml + 2 * (s * BHS + row));
-            if (ml[0] == -INFINITY) continue;
+        for (int s0 = 0; s0 < nsplit; s0 += LPR) {
+            const f2 ml = s0 == 0 ? ml0 : slice_ml(s0 + lane);
             const float w = __builtin_amdgcn_exp2f(ml[0] - M);
-            lsum += w * ml[1];
-            const f4 x = *reinterpret_cast<const f4 *>(a.part_o + (s * BHS + row) * HD + 4 * part);
+            lsum += (ml[0] == -INFINITY) ? 0.f : w * ml[1];
+            const int n = min(nsplit - s0, LPR);
+#pragma unroll 4
+            for (int s = grp; s < n; s += G) {
+                const float ws = __shfl(w, s, LPR);
+                const bool seen = __shfl(ml[0], s, LPR) != -INFINITY;   // (a slice that saw no key is left out)
+                const f4 x = *reinterpret_cast<const f4 *>(a.part_o + ((s0 + s) * BHS + row) * HD + 4 * part);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[j] += w * x[j];
+                for (int j = 0; j < 4; ++j) acc[j] += seen ? ws * x[j] : 0.f;
+            }
         }
+#pragma unroll
+        for (int off = 1; off < LPR; off <<= 1) lsum += __shfl_xor(lsum, off);
+#pragma unroll
+        for (int off = 16; off < LPR; off <<= 1)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[j] += __shfl_xor(acc[j], off);
     }
+    if (grp != 0) return;
     // inv_keep: 1/(1-p), which the slices left out of their O (1 without dropout).
     const float inv = lsum > 0.f ? a.inv_keep / lsum : 0.f;
 #pragma unroll
@@ -905,8 +932,7 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdArgs a) {
 // V from HBM once; an MFMA tile would use one of its 32 query rows.
 // ---------------------------------------------------------------------------
 // Workgroup (slice ks, b*H + h) takes the keys of slice ks (all keys when
-// nsplit = 1), cut into four runs of whole 64-key blocks, one per wave.  Per
-// block, lane L = 8g + c8 loads the 16-byte chunk c8 (dims 8*c8 .. +7) of key
+// nsplit = 1) in 64-key blocks, wave w blocks w, w + DEC_NW, ...  Per block, lane L = 8g + c8 loads the 16-byte chunk c8 (dims 8*c8 .. +7) of key
 // rows k0 + 8i + g, i = 0..7, of K and of V (each of the eight loads covers 1 KB
 // of consecutive rows), forms the partial dot of its chunk with q's, and a
 // butterfly over the 8 lanes of group g gives all of them the score of row
@@ -914,7 +940,22 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdArgs a) {
 // accumulates P V for its 8 dims.  The groups' states merge by shuffles (lanes
 // xor 8, 16, 32), the waves' in LDS; the result is O and LSE (nsplit = 1) or
 // the slice's partial for fwd_combine_kernel.
-constexpr int DEC_NW = 4;
+//
+// Bound by what one CU can keep in flight (57 GB/s per CU at most, whatever
+// the number of waves) and, with every CU at work, by HBM.  A wave holds one
+// block's rows in registers: the next block's K rows are requested as soon as
+// the scores have consumed this one's, its V rows after the P V sums.  Eight
+// waves per workgroup (four: 5-30% slower where a head has one workgroup,
+// sixteen: equal there, slower with many heads).
+//
+// STREAM: K and V by nontemporal loads, for a cache that takes more than a
+// third of the 256 MB Infinity Cache (DEC_STREAM_BYTES) and will not be there
+// at the next token: 70 -> 58.7 us at 403 MB (B*H = 96, Sk = 16384; 6.9 TB/s),
+// 19.8 -> 18.9 us at 101 MB.  Smaller caches can stay there and plain loads
+// are then as fast or faster (74 MB: 14.2 us against 14.7, 12.6 MB in one slice
+// 14.1 against 20.1).
+constexpr int DEC_NW = 8;
+constexpr int64_t DEC_STREAM_BYTES = 80 << 20;
 
 // Sum over the 8 lanes of each aligned group of 8, returned to all of them:
 // DPP quad_perm [1,0,3,2] and [2,3,0,1] (partners xor 1, xor 2), then
@@ -936,22 +977,19 @@ __device__ __forceinline__ void merge_state(float &m, float &l, f8 &acc, float m
     m = mx;
 }
 
-template <bool CAUSAL>
+template <bool CAUSAL, bool STREAM>
 __global__ __launch_bounds__(DEC_NW * 64) void decode_kernel(const FwdArgs a) {
     __shared__ float sm[DEC_NW][HD + 2];   // per wave: O accumulator, max, sum
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 3, c8 = lane & 7;
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 3, c8 = lane & 7;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int BH = a.B * a.H;
     const int ks = blockIdx.x / BH, bh = blockIdx.x - ks * BH;
     const int b = bh / a.H, h = bh - b * a.H;
     const int Sk = a.Sk;
     const int kend = CAUSAL ? min(Sk, a.coff + 1) : Sk;   // query 0 sees keys j <= coff
     const int kb = ks * a.split_keys, ke = min(kend, kb + a.split_keys);
-    const int nblk = ke > kb ? (ke - kb + 63) / 64 : 0;
-    const int per = (nblk + DEC_NW - 1) / DEC_NW;
-    const int wb = kb + 64 * min(nblk, wave * per);
-    const int we = min(ke, kb + 64 * min(nblk, (wave + 1) * per));
-    const _Float16 *Kp = a.k + b * a.ksb + h * a.ksh + 8 * c8;
-    const _Float16 *Vp = a.v + b * a.vsb + h * a.vsh + 8 * c8;
+    const _Float16 *Kp = a.k + b * a.ksb + h * a.ksh;
+    const _Float16 *Vp = a.v + b * a.vsb + h * a.vsh;
     const h8 qv = *reinterpret_cast<const h8 *>(a.q + b * a.qsb + h * a.qsh + 8 * c8);
     const h8 qn = neg_h8_if(qv, a.negate);
     const float scale2 = a.scale2;
@@ -960,25 +998,27 @@ __global__ __launch_bounds__(DEC_NW * 64) void decode_kernel(const FwdArgs a) {
     f8 acc;
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = 0.f;
-    // Block k0's rows are loaded while block k0 - 64 is computed (two register sets).
-    h8 kn[8], vn[8];
-    auto load = [&](int k0) FA2_INLINE {
+    h8 kx[8], vx[8];
+    // Rows k0 + 8i + g of K or V: a scalar base per block and 32-bit lane
+    // offsets (row strides are below 2^24 elements); rows past the cache's
+    // end read its last row (their scores are masked).
+    auto load = [&](const _Float16 *base, int64_t stride, int k0, h8(&x)[8]) FA2_INLINE {
+        const _Float16 *p = base + (int64_t)k0 * stride;
+        const uint32_t st = (uint32_t)stride;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const int r = min(k0 + 8 * i + g, Sk - 1);   // rows past the run: loaded in bounds, masked
-            kn[i] = *reinterpret_cast<const h8 *>(Kp + (int64_t)r * a.kss);
-            vn[i] = *reinterpret_cast<const h8 *>(Vp + (int64_t)r * a.vss);
+            const uint32_t r = (uint32_t)min(8 * i + g, Sk - 1 - k0);
+            const h8 *src = reinterpret_cast<const h8 *>(p + (mul_u24(st, r) + 8u * (uint32_t)c8));
+            x[i] = STREAM ? __builtin_nontemporal_load(src) : *src;
         }
     };
-    if (wb < we) load(wb);
-    for (int k0 = wb; k0 < we; k0 += 64) {
-        h8 kx[8], vx[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            kx[i] = kn[i];
-            vx[i] = vn[i];
-        }
-        if (k0 + 64 < we) load(k0 + 64);
+    int k0 = kb + 64 * wave;
+    if (k0 < ke) {
+        load(Kp, a.kss, k0, kx);
+        load(Vp, a.vss, k0, vx);
+    }
+    for (; k0 < ke; k0 += 64 * DEC_NW) {
+        const int kn = k0 + 64 * DEC_NW;
         float s[8];
         float mx = m;
 #pragma unroll
@@ -990,9 +1030,10 @@ __global__ __launch_bounds__(DEC_NW * 64) void decode_kernel(const FwdArgs a) {
                 d = __builtin_amdgcn_fdot2(qq, kk, d, false);
             }
             d = sum8(d);
-            s[i] = (k0 + 8 * i + g < we) ? d * scale2 : -INFINITY;
+            s[i] = (k0 + 8 * i + g < ke) ? d * scale2 : -INFINITY;
             mx = fmaxf(mx, s[i]);
         }
+        if (kn < ke) load(Kp, a.kss, kn, kx);
         const float alpha = (m == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m - mx);
         l *= alpha;
 #pragma unroll
@@ -1004,6 +1045,7 @@ __global__ __launch_bounds__(DEC_NW * 64) void decode_kernel(const FwdArgs a) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) acc[e] += p * (float)vx[i][e];
         }
+        if (kn < ke) load(Vp, a.vss, kn, vx);
         m = mx;
     }
     // Merge the 8 row groups (lanes with the same c8), then the waves.
@@ -1032,8 +1074,7 @@ __global__ __launch_bounds__(DEC_NW * 64) void decode_kernel(const FwdArgs a) {
 #pragma unroll
         for (int w = 0; w < DEC_NW; ++w) {
             const float mw = sm[w][HD];
-            if (mw == -INFINITY) continue;
-            const float wt = __builtin_amdgcn_exp2f(mw - M);
+            const float wt = (mw == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mw - M);
             L += wt * sm[w][HD + 1];
             o += wt * sm[w][lane];
         }
@@ -1144,25 +1185,35 @@ hipError_t launch_fwd(const FwdArgs &a, bool causal, bool dropout, hipStream_t s
     return hipGetLastError();
 }
 
+static hipError_t launch_combine(const FwdArgs &a, hipStream_t st) {
+    const int64_t rows = (int64_t)a.B * a.H * a.S;
+    if (a.nsplit > 4)
+        hipLaunchKernelGGL(fwd_combine_kernel<4>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL(fwd_combine_kernel<1>, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_fwd_decode(const FwdArgs &a, bool causal, hipStream_t st) {
     const dim3 grid((unsigned)(a.B * a.H * a.nsplit)), block(DEC_NW * 64);
-    if (causal)
-        hipLaunchKernelGGL(decode_kernel<true>, grid, block, 0, st, a);
+    const int64_t keys = causal ? std::max<int64_t>(0, std::min<int64_t>(a.Sk, (int64_t)a.coff + 1)) : a.Sk;   // read
+    const bool stream = (int64_t)a.B * a.H * keys * HD * 2 * (int64_t)sizeof(_Float16) > DEC_STREAM_BYTES;
+    if (causal && stream)
+        hipLaunchKernelGGL((decode_kernel<true, true>), grid, block, 0, st, a);
+    else if (causal)
+        hipLaunchKernelGGL((decode_kernel<true, false>), grid, block, 0, st, a);
+    else if (stream)
+        hipLaunchKernelGGL((decode_kernel<false, true>), grid, block, 0, st, a);
     else
-        hipLaunchKernelGGL(decode_kernel<false>, grid, block, 0, st, a);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || a.nsplit <= 1) return e;
-    hipLaunchKernelGGL(fwd_combine_kernel, dim3((unsigned)((a.B * a.H + 15) / 16)), dim3(256), 0, st, a);
-    return hipGetLastError();
+        hipLaunchKernelGGL((decode_kernel<false, false>), grid, block, 0, st, a);
+    const hipError_t e = hipGetLastError();
+    return (e != hipSuccess || a.nsplit <= 1) ? e : launch_combine(a, st);
 }
 
 hipError_t launch_fwd_split(const FwdArgs &a, bool causal, bool dropout, hipStream_t st) {
     launch_fwd_t<true>(a, causal, dropout, st);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const int64_t rows = (int64_t)a.B * a.H * a.S;
-    hipLaunchKernelGGL(fwd_combine_kernel, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, st, a);
-    return hipGetLastError();
+    return e != hipSuccess ? e : launch_combine(a, st);
 }
 
 }  // namespace fa2

@@ -147,11 +147,17 @@ int64_t auto_nsplit(int64_t wgs, int64_t tiles) {
     return std::max<int64_t>(1, std::min<int64_t>(384 / wgs, tiles / 8));
 }
 
-// Decode (one query, the VALU kernel, four waves per workgroup each taking a
-// quarter of its slice): about 192 workgroups and at least 1024 keys per
-// slice -- the best of a sweep over B*H = 12..384 and S_k = 1K..16K.
+// Decode (one query, the VALU kernel, one workgroup per head and slice): about
+// 192 workgroups and never more than one per CU (at B*H = 96 and S_k = 4096,
+// 192 workgroups take 20.6 us, 288 take 24.8 and 96 take 24.9), slices of at
+// least 256 keys, and none below 1536 keys, where the merge's launch costs
+// more than the slices save (B*H = 12: S_k = 1000 5.9 us in one piece, 7.6 in
+// two; S_k = 2500 10.3 in one, 8.4 in eight).
 int64_t auto_nsplit_decode(int64_t bh, int64_t s_k) {
-    return std::max<int64_t>(1, std::min<int64_t>((192 + bh - 1) / bh, s_k / 1024));
+    if (s_k < 1536) return 1;
+    int64_t n = (192 + bh - 1) / bh;
+    if (bh * n > 256) n = 256 / bh;
+    return std::max<int64_t>(1, std::min<int64_t>(n, s_k / 256));
 }
 
 std::vector<torch::Tensor> fa_fwd_kv(torch::Tensor q, torch::Tensor k, torch::Tensor v, bool causal,
