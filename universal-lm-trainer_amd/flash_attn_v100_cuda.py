@@ -176,10 +176,16 @@ def _fa_ready(t):
             and all((s * 2) % 32 == 0 for s in t.stride()[:3]))
 
 
+def _ready_bits(q, k, v):
+    """_fa_ready of q, k, v in bits 0..2 and, in bit 3, whether their shapes agree."""
+    if _EXT is not None:
+        return _EXT.ready3(q, k, v)
+    return (_fa_ready(q) | _fa_ready(k) << 1 | _fa_ready(v) << 2) | (q.shape == k.shape == v.shape) << 3
+
+
 def can_use(q, k, v):
     """Whether the tensors can go to the kernel directly (reference :105-108)."""
-    return (_fa_ready(q) and _fa_ready(k) and _fa_ready(v)
-            and q.shape == k.shape == v.shape)
+    return _ready_bits(q, k, v) == 15
 
 
 class _RopeV100Cuda(torch.autograd.Function):
@@ -228,8 +234,9 @@ def flash_attn_v100(q, k, v, dropout_p: float = 0.0, causal: bool = True, softma
     """Causal FlashAttention-2 on MI355X; same contract as the reference (:155-166)."""
     if not (q.is_cuda and q.dtype == torch.float16 and q.size(3) == 64):
         raise ValueError("flash_attn_v100 only supports fp16 GPU tensors with head_dim=64")
-    if not _fa_ready(q) or not _fa_ready(k) or not _fa_ready(v):
-        q, k, v = (t if _fa_ready(t) else t.contiguous() for t in (q, k, v))
+    ready = _ready_bits(q, k, v)
+    if ready & 7 != 7:
+        q, k, v = (t if ready >> i & 1 else t.contiguous() for i, t in enumerate((q, k, v)))
     if softmax_scale is None:
         softmax_scale = q.shape[-1] ** -0.5
     return _FlashAttnV100Cuda.apply(q, k, v, float(dropout_p), bool(causal), float(softmax_scale))
@@ -245,7 +252,7 @@ def _needs_grad(*ts):
 
 def _kv_ready(q, k, v):
     """fp16 (B,H,S_q,64) queries against (B,H,S_k,64) keys/values, kernel-aligned."""
-    return (_fa_ready(q) and _fa_ready(k) and _fa_ready(v) and k.shape == v.shape
+    return (_ready_bits(q, k, v) & 7 == 7 and k.shape == v.shape
             and k.shape[:2] == q.shape[:2] and k.size(2) >= 1)
 
 
@@ -254,9 +261,11 @@ def _fwd_kv(q, k, v, causal, softmax_scale, causal_offset):
         raise ValueError("fp16 GPU tensors (B,H,S,64) only")
     if _needs_grad(q, k, v):
         raise RuntimeError("the key/value-length forward is inference-only (no backward)")
-    q, k, v = (t if _fa_ready(t) else t.contiguous() for t in (q, k, v))
+    ready = _ready_bits(q, k, v)
+    if ready & 7 != 7:
+        q, k, v = (t if ready >> i & 1 else t.contiguous() for i, t in enumerate((q, k, v)))
     if softmax_scale is None:
-        softmax_scale = q.shape[-1] ** -0.5
+        softmax_scale = 0.125   # 64 ** -0.5
     o, _ = extension().fa_fwd_kv(q, k, v, bool(causal), float(softmax_scale), int(causal_offset))
     return o
 
