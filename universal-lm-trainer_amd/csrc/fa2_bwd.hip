@@ -489,7 +489,7 @@ __global__ __launch_bounds__(256, NARROW ? DQ_NARROW_WAVES : 2) void bwd_dq_pipe
                              : reinterpret_cast<char *>(sKV[stage_of(ntiles + (wave >> 1))]) + 8192 * (wave & 1);
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb)
-        store_rows_f16(dq[qb][0], dq[qb][1], sc, stg + 4096 * qb, dQp + (int64_t)(qw0 + 32 * qb) * a.dqss, a.dqss,
+        store_rows_f16<true>(dq[qb][0], dq[qb][1], sc, stg + 4096 * qb, dQp + (int64_t)(qw0 + 32 * qb) * a.dqss, a.dqss,
                        S - (qw0 + 32 * qb), dq16);
 }
 
@@ -919,9 +919,9 @@ __device__ __forceinline__ void dkv_block(const BwdArgs &a, const int kblk, cons
     static_assert(sizeof(sQD) >= KP_NW * 8192, "dK/dV staging fits in the stages");
     const float sc = a.scale;
     char *const stg = reinterpret_cast<char *>(&sQD[0][0][0]) + 8192 * wave;
-    store_rows_f16(dk[0], dk[1], sc, stg, dKp + (int64_t)kw0 * a.dkss, a.dkss, S - kw0,
+    store_rows_f16<true>(dk[0], dk[1], sc, stg, dKp + (int64_t)kw0 * a.dkss, a.dkss, S - kw0,
                    ((a.dksb | a.dksh | a.dkss) & 7) == 0);
-    store_rows_f16(dv[0], dv[1], 1.f, stg + 4096, dVp + (int64_t)kw0 * a.dvss, a.dvss, S - kw0,
+    store_rows_f16<true>(dv[0], dv[1], 1.f, stg + 4096, dVp + (int64_t)kw0 * a.dvss, a.dvss, S - kw0,
                    ((a.dvsb | a.dvsh | a.dvss) & 7) == 0);
 }
 

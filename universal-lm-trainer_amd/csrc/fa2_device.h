@@ -302,7 +302,14 @@ __device__ __forceinline__ float xor32(float x) { return __shfl_xor(x, 32); }
 // chunk ch at chunk ch ^ (r & 7): the row reads are conflict-free, the
 // 8-byte writes put rows 8 apart on the same banks), and leaves as
 // whole 128-byte rows, 8 lanes x 16 bytes (8-byte halves unless `vec16`:
-// dst and stride multiples of 8 elements).
+// dst and stride multiples of 8 elements).  STREAM: the rows leave by
+// nontemporal stores, which take no place in the L2 from the tiles the grid is
+// reading; the gradients use it (forward and backward of B=64 H=12 S=512 237.6
+// -> 223.7 us, B=31 S=1050 363.7 -> 352, B=16 S=2048 541 -> 533, B=8 S=4096 951
+// -> 942; with elementwise readers of all outputs following still 3%, 1.5%,
+// 0.9% and 0.4% faster).  O, which the backward reads again, does not (with it
+// streamed too, B=4 S=4096 and its readers took 0.7% longer).
+template <bool STREAM = false>
 __device__ __forceinline__ void store_rows_f16(const f16x &acc0, const f16x &acc1, float mul, char *blk,
                                                _Float16 *dst, int64_t stride, int nrows, bool vec16) {
     const int lane = threadIdx.x & 63, c = lane & 31, g2 = lane >> 5;
@@ -324,7 +331,10 @@ __device__ __forceinline__ void store_rows_f16(const f16x &acc0, const f16x &acc
         if (r < nrows) {
             _Float16 *p = dst + r * stride + 8 * ch;
             if (vec16) {
-                *reinterpret_cast<h8 *>(p) = v;
+                if (STREAM)
+                    __builtin_nontemporal_store(v, reinterpret_cast<h8 *>(p));
+                else
+                    *reinterpret_cast<h8 *>(p) = v;
             } else {
                 *reinterpret_cast<h4 *>(p) = __builtin_shufflevector(v, v, 0, 1, 2, 3);
                 *reinterpret_cast<h4 *>(p + 4) = __builtin_shufflevector(v, v, 4, 5, 6, 7);
