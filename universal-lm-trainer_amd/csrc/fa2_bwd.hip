@@ -990,6 +990,9 @@ hipError_t launch_bwd_delta(const BwdArgs &a, hipStream_t st) {
 // Workgroup order of the dQ pass (query_block_order): groups of 16 heads per
 // XCD up to this length (measured at B*S = 32k, H = 12: S = 512 3.5% faster;
 // S = 1024 4.5% and S = 2048 11% slower), the plain order beyond.
+// Not with dropout: the two-block kernel of the keep words has half the
+// workgroups and needs the plain order's packing (B=12 H=16 S=512 35.0 -> 26.8
+// us, B=40 H=16 S=300 52.0 -> 46.8, B=64 H=12 S=512 equal).
 #ifndef FA2_DQ_GROUP_MAX_S
 #define FA2_DQ_GROUP_MAX_S 512
 #endif
@@ -997,7 +1000,7 @@ hipError_t launch_bwd_delta(const BwdArgs &a, hipStream_t st) {
 template <bool NARROW>
 static void launch_dq_t(const BwdArgs &a_in, bool causal, bool dropout, hipStream_t st) {
     BwdArgs a = a_in;
-    a.hgroup = (a.B * a.H) % 8 == 0 && a.S <= FA2_DQ_GROUP_MAX_S ? 16 : 0;
+    a.hgroup = !dropout && (a.B * a.H) % 8 == 0 && a.S <= FA2_DQ_GROUP_MAX_S ? 16 : 0;
     const int qwg = NARROW && !(dropout && a.drop_mask != nullptr) ? DQ_NW * 32 : DQ_QWG;
     const dim3 grid((unsigned)((a.S + qwg - 1) / qwg * a.B * a.H)), block(256);
     a.qbase = query_block_base(causal, a.S, qwg, grid.x, (int64_t)(qwg == DQ_QWG ? 2 : DQ_NARROW_WAVES) * device_cus());

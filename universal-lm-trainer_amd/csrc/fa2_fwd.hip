@@ -1105,6 +1105,10 @@ void launch_narrow(const FwdArgs &a, hipStream_t st) {
 // head's K / V tiles would otherwise leave the L2 between its query blocks
 // (measured at B*S = 32k, H = 12: S = 512 9% faster, S = 1024 5%; S = 2048
 // 2% slower, S = 4096 equal); the plain order otherwise.
+// With dropout the hash bounds the kernel, not its tiles, and the plain order,
+// heaviest query blocks first over the whole grid, packs the slots better
+// (H = 12, p = 0.1, with keep words: B=16 S=1024 70.3 -> 63.5 us, B=32 S=700
+// 70.4 -> 64.6, B=64 S=512 79.5 -> 76.6).
 #ifndef FA2_FWD_GROUP_MAX_S
 #define FA2_FWD_GROUP_MAX_S 1024
 #endif
@@ -1126,7 +1130,7 @@ void launch_fwd_t(const FwdArgs &a_in, bool causal, bool dropout, hipStream_t st
     // was 5-16% slower there).
     const int64_t narrow_wgs = (int64_t)((a.S + qwg_of(1) - 1) / qwg_of(1)) * a.B * a.H;
     if (!SPLIT && FA2_FWD_NARROW && narrow_wgs >= (int64_t)NARROW_WAVES * device_cus()) {
-        if ((a.B * a.H) % 8 == 0 && a.S <= FA2_FWD_GROUP_MAX_S) a.hgroup = 16;
+        if (!dropout && (a.B * a.H) % 8 == 0 && a.S <= FA2_FWD_GROUP_MAX_S) a.hgroup = 16;
         a.qbase = query_block_base(causal, a.S, qwg_of(1), narrow_wgs, (int64_t)NARROW_WAVES * device_cus());
         if (causal) {
             if (dmask) launch_narrow<true, true, true>(a, st);
