@@ -46,3 +46,35 @@ def test_partial_first_query_block(fa, B, H, S, p):
         assert orc.max_abs(got[0], ro) <= 2e-3 / (1.0 - p) and orc.max_abs(got[1], rl) <= 1e-3
         for name, a, r in zip(("dQ", "dK", "dV"), got[2:], rg):
             assert orc.rel_l2(a, r) <= 1e-2, (name, b, h)
+
+
+@pytest.mark.parametrize("B,H,S,causal", [(43, 3, 140, True),    # 129 heads, numbered as 136: grouped orders
+                                          (33, 4, 1100, True),   # 132 heads: plain forward, two-block dQ
+                                          (43, 3, 150, False)])
+def test_padded_head_numbers(fa, B, H, S, causal):
+    """B*H no multiple of 8 from 128 heads on: every head of every output is written and gives the bits
+    it gives alone in a small batch (up to 127 heads the grid numbers the heads as they are); the forward
+    loops and both dQ kernels agree bit for bit."""
+    print(f"case padded heads B={B} H={H} S={S} causal={causal}", flush=True)
+    ext = fa.extension()
+    g = torch.Generator().manual_seed(B * S)
+    q, k, v, do = (torch.randn(B, H, S, 64, generator=g).half().to(DEV) for _ in range(4))
+    for p in (0.0, 0.1):
+        for _ in range(6):
+            torch.full_like(q, float("nan"))
+        o, lse = ext.fa_fwd(q, k, v, p, causal, 0.125, 5)
+        outs = (o, lse, *ext.fa_bwd(q, k, v, o, lse, do, p, causal, 0.125, 5, 7))
+        for t in outs:
+            assert torch.isfinite(t).all()
+        n = 5   # the first batches alone (the dropout hash numbers heads from 0 in both calls)
+        a = [t[:n].contiguous() for t in (q, k, v, do)]
+        o1, l1 = ext.fa_fwd(*a[:3], p, causal, 0.125, 5)
+        alone = (o1, l1, *ext.fa_bwd(*a[:3], o1, l1, a[3], p, causal, 0.125, 5, 7))
+        for x, y in zip(outs, alone):
+            assert torch.equal(x[:n], y)
+        if p == 0:   # and the last batches, whose workgroups sit beside the ones with no head
+            a = [t[-n:].contiguous() for t in (q, k, v, do)]
+            o1, l1 = ext.fa_fwd(*a[:3], p, causal, 0.125, 5)
+            alone = (o1, l1, *ext.fa_bwd(*a[:3], o1, l1, a[3], p, causal, 0.125, 5, 7))
+            for x, y in zip(outs, alone):
+                assert torch.equal(x[-n:], y)

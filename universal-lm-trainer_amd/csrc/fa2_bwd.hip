@@ -129,7 +129,8 @@ __global__ __launch_bounds__(256, NARROW ? DQ_NARROW_WAVES : 2) void bwd_dq_pipe
     const int BH = a.B * a.H;
     const int nqblk = (S + QWG - 1) / QWG;
     int qslot, bh;
-    query_block_order(blockIdx.x, BH, nqblk, a.hgroup, qslot, bh);
+    query_block_order(blockIdx.x, a.bhp, nqblk, a.hgroup, qslot, bh);
+    if (bh >= BH) return;
     const int qblk = nqblk - 1 - qslot;   // heaviest (last) query blocks first
     const int b = bh / a.H, h = bh - b * a.H;
 
@@ -947,8 +948,9 @@ __global__ __launch_bounds__(256, 2) void bwd_dkv_pipe_kernel(const BwdArgs a) {
         bh = 8 * (i / nwg_head) + xcd;
         j = i - (i / nwg_head) * nwg_head;
     } else {
-        j = L / BH;
-        bh = L - j * BH;
+        j = L / a.bhp;
+        bh = L - j * a.bhp;
+        if (bh >= BH) return;
     }
     // Single blocks: j = 0, the heaviest under the causal mask, first.  Pairs
     // of short blocks (nkb <= 8: S <= 1024): every other workgroup runs its
@@ -1000,9 +1002,9 @@ hipError_t launch_bwd_delta(const BwdArgs &a, hipStream_t st) {
 template <bool NARROW>
 static void launch_dq_t(const BwdArgs &a_in, bool causal, bool dropout, hipStream_t st) {
     BwdArgs a = a_in;
-    a.hgroup = !dropout && (a.B * a.H) % 8 == 0 && a.S <= FA2_DQ_GROUP_MAX_S ? 16 : 0;
+    a.hgroup = !dropout && a.bhp % 8 == 0 && a.S <= FA2_DQ_GROUP_MAX_S ? 16 : 0;
     const int qwg = NARROW && !(dropout && a.drop_mask != nullptr) ? DQ_NW * 32 : DQ_QWG;
-    const dim3 grid((unsigned)((a.S + qwg - 1) / qwg * a.B * a.H)), block(256);
+    const dim3 grid((unsigned)((a.S + qwg - 1) / qwg * a.bhp)), block(256);
     a.qbase = query_block_base(causal, a.S, qwg, grid.x, (int64_t)(qwg == DQ_QWG ? 2 : DQ_NARROW_WAVES) * device_cus());
     const bool dmask = dropout && a.drop_mask != nullptr;
     if (causal) {
@@ -1041,7 +1043,7 @@ hipError_t launch_bwd_dkv(const BwdArgs &a_in, bool causal, bool dropout, hipStr
     const int64_t xcd_slots = 2 * (int64_t)device_cus() / 8;
     a.dkv_pair = causal && !dropout && bh % 8 == 0 && per_xcd > 0 && per_xcd % xcd_slots == 0;
     const int nwg = a.dkv_pair ? (nkblk + 1) / 2 : nkblk;
-    const dim3 grid((unsigned)(nwg * a.B * a.H)), block(256);
+    const dim3 grid((unsigned)(nwg * (a.dkv_pair ? a.B * a.H : a.bhp))), block(256);
     // The folded row terms need -lse2/scale2 finite (|lse2| < 3e18 at this bound).
     const bool fold = !dropout && a.scale2 >= 1e-20f;
     const bool dmask = dropout && a.drop_mask != nullptr;

@@ -446,27 +446,28 @@ __device__ __forceinline__ int64_t dmask_word(bool causal, int bh, int S, int t6
 }
 
 // Workgroup order of the query-block kernels (forward, dQ pass): workgroup L
-// of a grid of nq * BH -> its query slot (0 = the head's last, heaviest
-// query block) and its head bh.  Workgroups go to the 8 XCDs in turn
-// (L % 8), each XCD with its own L2.
-//   * G = 0: query slots outermost, heads fastest.  With BH a multiple of 8
+// of a grid of nq * BHP -> its query slot (0 = the head's last, heaviest
+// query block) and its head bh, which for the BHP - B*H numbers added to the
+// heads (grid_heads) is past the last one: nothing to do.  Workgroups go to
+// the 8 XCDs in turn (L % 8), each XCD with its own L2.
+//   * G = 0: query slots outermost, heads fastest.  With BHP a multiple of 8
 //     a head's workgroups share one XCD, heaviest first over the whole grid,
-//     but BH workgroups apart in time.
-//   * G > 0 (the host passes it only when BH is a multiple of 8): XCD x takes
+//     but BHP workgroups apart in time.
+//   * G > 0 (the host passes it only when BHP is a multiple of 8): XCD x takes
 //     the heads x + 8 y and runs them in groups of G heads, query slots
 //     heaviest first within each group, so that the query blocks of a head
 //     run at about the same time and share its K / V tiles in the XCD's L2.
-__device__ __forceinline__ void query_block_order(int L, int BH, int nq, int G, int &qslot, int &bh) {
+__device__ __forceinline__ void query_block_order(int L, int BHP, int nq, int G, int &qslot, int &bh) {
     if (G > 0) {
         const int xcd = L & 7, i = L >> 3;
-        const int per = G * nq;                       // workgroups of a full group
+        const int per = G * nq;                        // workgroups of a full group
         const int grp = i / per, r = i - grp * per;
-        const int gsz = min(G, (BH >> 3) - grp * G);  // the last group may be smaller
+        const int gsz = min(G, (BHP >> 3) - grp * G);  // the last group may be smaller
         qslot = r / gsz;
         bh = 8 * (grp * G + r - qslot * gsz) + xcd;
     } else {
-        qslot = L / BH;
-        bh = L - qslot * BH;
+        qslot = L / BHP;
+        bh = L - qslot * BHP;
     }
 }
 

@@ -133,7 +133,8 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
         ks = rem / BH;
         bh = rem - ks * BH;
     } else {
-        query_block_order(L, BH, nqblk, a.hgroup, qslot, bh);
+        query_block_order(L, a.bhp, nqblk, a.hgroup, qslot, bh);
+        if (bh >= BH) return;
     }
     const int qblk = nqblk - 1 - qslot;                // heaviest (last) query blocks first
     const int b = bh / a.H, h = bh - b * a.H;
@@ -1096,7 +1097,7 @@ __global__ __launch_bounds__(DEC_NW * 64) void decode_kernel(const FwdArgs a) {
 template <bool CAUSAL, bool DROPOUT, bool DMASK>
 void launch_narrow(const FwdArgs &a, hipStream_t st) {
     const int nqblk = (a.S + qwg_of(1) - 1) / qwg_of(1);
-    hipLaunchKernelGGL((fwd_kernel<CAUSAL, DROPOUT, false, DMASK, 1, true>), dim3((unsigned)(nqblk * a.B * a.H)),
+    hipLaunchKernelGGL((fwd_kernel<CAUSAL, DROPOUT, false, DMASK, 1, true>), dim3((unsigned)(nqblk * a.bhp)),
                        dim3(NW * 64), 0, st, a);
 }
 
@@ -1130,7 +1131,7 @@ void launch_fwd_t(const FwdArgs &a_in, bool causal, bool dropout, hipStream_t st
     // was 5-16% slower there).
     const int64_t narrow_wgs = (int64_t)((a.S + qwg_of(1) - 1) / qwg_of(1)) * a.B * a.H;
     if (!SPLIT && FA2_FWD_NARROW && narrow_wgs >= (int64_t)NARROW_WAVES * device_cus()) {
-        if (!dropout && (a.B * a.H) % 8 == 0 && a.S <= FA2_FWD_GROUP_MAX_S) a.hgroup = 16;
+        if (!dropout && a.bhp % 8 == 0 && a.S <= FA2_FWD_GROUP_MAX_S) a.hgroup = 16;
         a.qbase = query_block_base(causal, a.S, qwg_of(1), narrow_wgs, (int64_t)NARROW_WAVES * device_cus());
         if (causal) {
             if (dmask) launch_narrow<true, true, true>(a, st);
@@ -1152,7 +1153,7 @@ void launch_fwd_t(const FwdArgs &a_in, bool causal, bool dropout, hipStream_t st
     const bool two = !SPLIT && !dmask &&
                      (int64_t)((a.S + qwg_of(2) - 1) / qwg_of(2)) * a.B * a.H >= 2 * (int64_t)device_cus();
     const int nqblk = (a.S + (two ? qwg_of(2) : qwg_of(1)) - 1) / (two ? qwg_of(2) : qwg_of(1));
-    const dim3 grid((unsigned)(nqblk * a.B * a.H * (SPLIT ? a.nsplit : 1)));
+    const dim3 grid((unsigned)(SPLIT ? nqblk * a.B * a.H * a.nsplit : nqblk * a.bhp));
     if (!SPLIT)
         a.qbase = query_block_base(causal, a.S, two ? qwg_of(2) : qwg_of(1), grid.x, 2 * (int64_t)device_cus());
     if (causal) {
