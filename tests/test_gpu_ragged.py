@@ -78,3 +78,20 @@ def test_padded_head_numbers(fa, B, H, S, causal):
             alone = (o1, l1, *ext.fa_bwd(*a[:3], o1, l1, a[3], p, causal, 0.125, 5, 7))
             for x, y in zip(outs, alone):
                 assert torch.equal(x[-n:], y)
+
+
+@pytest.mark.parametrize("S,causal", [(1025, True), (1300, False), (2100, True)])
+def test_narrow_dq_on_small_long_grids(fa, S, causal):
+    """Longer sequences whose two-block dQ grid leaves slots empty take the narrow kernel: a few heads
+    give the bits that the same heads give in a batch large enough for the two-block kernel."""
+    print(f"case small long dQ grid S={S} causal={causal}", flush=True)
+    ext = fa.extension()
+    g = torch.Generator().manual_seed(S)
+    B = 520 // ((S + 255) // 256 * 4) + 1   # more than 15/16 of 512 two-block workgroups at H = 4
+    q, k, v, do = (torch.randn(B, 4, S, 64, generator=g).half().to(DEV) for _ in range(4))
+    for p in (0.0, 0.1):
+        o, lse = ext.fa_fwd(q, k, v, p, causal, 0.125, 9)
+        big = ext.fa_bwd(q, k, v, o, lse, do, p, causal, 0.125, 9, 7)
+        small = ext.fa_bwd(q[:2], k[:2], v[:2], o[:2], lse[:2], do[:2], p, causal, 0.125, 9, 7)
+        for x, y in zip(big, small):
+            assert torch.equal(x[:2], y)

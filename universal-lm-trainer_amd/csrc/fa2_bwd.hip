@@ -1025,7 +1025,13 @@ static void launch_dq_t(const BwdArgs &a_in, bool causal, bool dropout, hipStrea
 }
 
 hipError_t launch_bwd_dq(const BwdArgs &a, bool causal, bool dropout, hipStream_t st) {
-    if (a.S <= FA2_DQ_NARROW_MAX_S)
+    // Longer sequences whose two-block grid leaves slots empty (at most 15/16 of
+    // two workgroups per CU) take the narrow kernel too, for twice the
+    // workgroups and the same bits: H = 12, B=1 S=4096 93.1 -> 69.0 us, B=2
+    // S=4096 108.4 -> 93.4, B=2 S=2730 68.5 -> 53.0, B=5 S=2048 (480 workgroups)
+    // 66.1 -> 59.3; B=7 S=1500 (504) 52.3 -> 53.7, so not there.
+    const int64_t two_wgs = (int64_t)((a.S + DQ_QWG - 1) / DQ_QWG) * a.B * a.H;
+    if (a.S <= FA2_DQ_NARROW_MAX_S || 16 * two_wgs <= 15 * 2 * (int64_t)device_cus())
         launch_dq_t<true>(a, causal, dropout, st);
     else
         launch_dq_t<false>(a, causal, dropout, st);
