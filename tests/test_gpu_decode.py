@@ -60,3 +60,18 @@ def test_decode_merge_edges(fa):
     for nsplit in (1, 4):
         o, lse = ext.fa_fwd_kv(q, k, v, True, 0.125, -1, nsplit)
         assert (o == 0).all() and (lse == float("-inf")).all(), nsplit
+
+
+@pytest.mark.parametrize("op,BH", [("decode", (1 << 23) + 3), ("forward", (1 << 24) - 1)])
+def test_many_heads_of_one_key(fa, op, BH):
+    """More heads than one launch of eight-wave decode workgroups can number, and the most the forward's
+    grid can: with one key, O is V and LSE the score."""
+    print(f"case one key op={op} BH={BH}", flush=True)
+    g = torch.Generator(DEV).manual_seed(1)
+    q, k, v = (torch.randn(1, BH, 1, 64, generator=g, device=DEV, dtype=torch.float16) for _ in range(3))
+    ext = fa.extension()
+    o, lse = ext.fa_fwd_kv(q, k, v, True, 0.125, 0, 0) if op == "decode" else ext.fa_fwd(q, k, v, 0.0, True, 0.125, 0)
+    assert torch.equal(o, v)
+    for part in (slice(0, 1000), slice((1 << 22) - 500, (1 << 22) + 500), slice(BH - 1000, BH)):
+        s = (q[0, part, 0].float() * k[0, part, 0].float()).sum(-1) * 0.125
+        assert (lse[0, part, 0] - s).abs().max().item() <= 1e-3

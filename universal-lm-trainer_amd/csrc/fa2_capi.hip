@@ -221,6 +221,7 @@ static int fwd_common(const fa2_fwd_params *p, int32_t s_k, int32_t coff, void *
     a.hgroup = 0;
     a.qbase = 0;
     a.bhp = fa2::grid_heads((int64_t)p->B * p->H);
+    a.wg0 = 0;
     const hipStream_t st = (hipStream_t)stream;
     const hipError_t e = (inference && p->S == 1 && !dropout) ? fa2::launch_fwd_decode(a, causal, st)
                          : nsplit > 1                         ? fa2::launch_fwd_split(a, causal, dropout, st)

@@ -984,7 +984,8 @@ __global__ __launch_bounds__(DEC_NW * 64) void decode_kernel(const FwdArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 3, c8 = lane & 7;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int BH = a.B * a.H;
-    const int ks = blockIdx.x / BH, bh = blockIdx.x - ks * BH;
+    const int wg = a.wg0 + (int)blockIdx.x;
+    const int ks = wg / BH, bh = wg - ks * BH;
     const int b = bh / a.H, h = bh - b * a.H;
     const int Sk = a.Sk;
     const int kend = CAUSAL ? min(Sk, a.coff + 1) : Sk;   // query 0 sees keys j <= coff
@@ -1192,26 +1193,35 @@ hipError_t launch_fwd(const FwdArgs &a, bool causal, bool dropout, hipStream_t s
 
 static hipError_t launch_combine(const FwdArgs &a, hipStream_t st) {
     const int64_t rows = (int64_t)a.B * a.H * a.S;
-    if (a.nsplit > 4)
+    // (64 threads a query reach the launch limit of 2^32 threads at 2^26.)
+    if (a.nsplit > 4 && rows < (1 << 26) - 4)
         hipLaunchKernelGGL(fwd_combine_kernel<4>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, a);
     else
         hipLaunchKernelGGL(fwd_combine_kernel<1>, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
+template <bool CAUSAL, bool STREAM>
+static hipError_t launch_decode(const FwdArgs &a_in, hipStream_t st) {
+    FwdArgs a = a_in;
+    // 2^22 workgroups per launch at most: the launch limit of 2^32 threads is
+    // 2^23 of eight waves, and B*H may be more.
+    const int64_t wgs = (int64_t)a.B * a.H * a.nsplit, per = 1 << 22;
+    for (int64_t w = 0; w < wgs; w += per) {
+        a.wg0 = (int)w;
+        hipLaunchKernelGGL((decode_kernel<CAUSAL, STREAM>), dim3((unsigned)std::min(per, wgs - w)), dim3(DEC_NW * 64),
+                           0, st, a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 hipError_t launch_fwd_decode(const FwdArgs &a, bool causal, hipStream_t st) {
-    const dim3 grid((unsigned)(a.B * a.H * a.nsplit)), block(DEC_NW * 64);
     const int64_t keys = causal ? std::max<int64_t>(0, std::min<int64_t>(a.Sk, (int64_t)a.coff + 1)) : a.Sk;   // read
     const bool stream = (int64_t)a.B * a.H * keys * HD * 2 * (int64_t)sizeof(_Float16) > DEC_STREAM_BYTES;
-    if (causal && stream)
-        hipLaunchKernelGGL((decode_kernel<true, true>), grid, block, 0, st, a);
-    else if (causal)
-        hipLaunchKernelGGL((decode_kernel<true, false>), grid, block, 0, st, a);
-    else if (stream)
-        hipLaunchKernelGGL((decode_kernel<false, true>), grid, block, 0, st, a);
-    else
-        hipLaunchKernelGGL((decode_kernel<false, false>), grid, block, 0, st, a);
-    const hipError_t e = hipGetLastError();
+    const hipError_t e = causal ? (stream ? launch_decode<true, true>(a, st) : launch_decode<true, false>(a, st))
+                                : (stream ? launch_decode<false, true>(a, st) : launch_decode<false, false>(a, st));
     return (e != hipSuccess || a.nsplit <= 1) ? e : launch_combine(a, st);
 }
 

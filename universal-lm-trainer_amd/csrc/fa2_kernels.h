@@ -35,6 +35,7 @@ struct FwdArgs {
     int hgroup;
     int qbase;           // first query of query block 0 (query_block_base)
     int bhp;             // head numbers of the grid (grid_heads)
+    int wg0;             // decode: number of the launch's first workgroup
 };
 
 struct BwdArgs {
@@ -109,8 +110,10 @@ inline int query_block_base(bool causal, int S, int qwg, int64_t wgs, int64_t sl
 // then go in groups, query_block_order); forward and backward of B=13 S=1100
 // without the causal mask 289 -> 276, B=11 S=2800 680 -> 668.  From 128 heads
 // on: with fewer, the XCDs with one head more set the time (108 heads at
-// S = 1500: dQ pass 67 -> 71 us).
-inline int grid_heads(int64_t bh) { return (int)(bh >= 128 ? (bh + 7) & ~(int64_t)7 : bh); }
+// S = 1500: dQ pass 67 -> 71 us).  Not from 2^20 heads on: the rounding gains
+// nothing there and could reach the launch limit of 2^32 threads, which
+// 2^24 - 1 heads of one block keep below.
+inline int grid_heads(int64_t bh) { return (int)(bh >= 128 && bh < (1 << 20) ? (bh + 7) & ~(int64_t)7 : bh); }
 
 // Compute units of the current device (cached per device; 256 on MI355X).
 // Launchers use it to size grids against the slots of two workgroups per CU.
