@@ -46,6 +46,49 @@ def test_decode_many_slices(fa, nsplit):
     assert (lse - rl).abs().max().item() <= 1e-3
 
 
+def split_inputs(H, Sq, Sk):
+    """q, k and V with a mean of 1: O is about 1 and a slice left out of n shows as 1/n of it."""
+    g = torch.Generator().manual_seed(Sk)
+    q = torch.randn(1, H, Sq, 64, generator=g).half().to(DEV)
+    k, v = (torch.randn(1, H, Sk, 64, generator=g).add(m).half().to(DEV) for m in (0.0, 1.0))
+    return q, k, v
+
+
+@pytest.mark.parametrize("Sq", [1, 5])
+@pytest.mark.parametrize("lo", [1, 65, 129])
+def test_merge_every_slice_count(fa, Sq, lo):
+    """64 slice counts from lo on, every slice one 64-key tile that all queries see: the groups of 16
+    lanes that share a query's slices end up with every possible remainder.  O against the reference
+    (the smallest share is about 1/192, more than twice O_TOL)."""
+    print(f"case slice counts {lo}..{lo + 63} Sq={Sq}", flush=True)
+    ext = fa.extension()
+    q, k, v = split_inputs(2, Sq, 64 * (lo + 63))
+    for n in range(lo, lo + 64):
+        kk, vv = k[:, :, :64 * n], v[:, :, :64 * n]
+        o, lse = ext.fa_fwd_kv(q, kk, vv, False, 0.125, 0, n)
+        ro, rl = reference(q, kk, vv, 64 * n)
+        assert (o.float() - ro).abs().max().item() <= O_TOL, n
+        assert (lse - rl).abs().max().item() <= 1e-3, n
+
+
+@pytest.mark.parametrize("H,Sq,Sk,slices", [(8, 1, 4352, 17), (4, 1, 5376, 21), (8, 1, 5376, 21), (4, 1, 8448, 33),
+                                            (4, 1, 8704, 34), (1, 1, 16128, 63), (4, 128, 8704, 17),
+                                            (12, 128, 8704, 17), (6, 300, 10752, 21)])
+def test_merge_of_automatic_slices(fa, H, Sq, Sk, slices):
+    """Calls through the public entry point whose automatic slice count is no multiple of four."""
+    print(f"case automatic slices H={H} Sq={Sq} Sk={Sk}", flush=True)
+    q, k, v = split_inputs(H, Sq, Sk)
+    o = fa.flash_attn_kvcache(q, k, v, causal=True)
+    ext = fa.extension()
+    for nsplit, tol in ((slices, 0.0), (1, O_TOL)):   # the count the rule takes, and the unsplit pass
+        assert (o - ext.fa_fwd_kv(q, k, v, True, 0.125, Sk - Sq, nsplit)[0]).abs().max().item() <= tol, nsplit
+    rows = torch.arange(Sq, device=DEV)[:, None] + (Sk - Sq)
+    s = torch.matmul(q.float(), k.float().transpose(-1, -2).contiguous()) * 0.125
+    s.masked_fill_(torch.arange(Sk, device=DEV)[None, :] > rows, float("-inf"))
+    ro = torch.matmul(torch.softmax(s, dim=-1), v.float())
+    assert (o.float() - ro).abs().max().item() <= O_TOL
+
+
 def test_decode_merge_edges(fa):
     """The merge of slices gives NaN where a slice's softmax met an infinite score (inf - inf), and a
     query that sees no key gives O = 0 and LSE = -inf with one slice and with several."""

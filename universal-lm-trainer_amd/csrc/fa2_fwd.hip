@@ -871,10 +871,15 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
 // and LSE = (M + log2 sum_s w_s l_s) ln 2 (a query no slice saw: O = 0,
 // LSE = -inf).  G groups of 16 lanes per query: each lane reads one slice's
 // max and sum (16 G slices at a time), then group g takes slices g, g + G, ...,
-// 4 of the 64 columns per lane, so that no load waits for another slice's.
-// Latency bound (3.8 us for a few rows, launch included): G = 4 from five
-// slices on (16 slices of 12 rows 6.1 -> 3.9 us, 8 slices of 3072 rows
-// 5.9 -> 4.1), G = 1 for fewer, where the rows alone fill the card.
+// 4 of the 64 columns per lane.  All groups run the same steps, the last one
+// on clamped slices of weight 0: the weights are read from other groups' lanes,
+// and a lane that has left the loop would give 0 for them.
+// Latency bound, so each step has four slices' loads in flight, the first
+// step's ahead of the maxima.  With the split forward before it, against lanes
+// that walk the slices one by one: 12 rows of 16 slices 15.6 -> 9.1 us, of 64
+// 40 -> 9.7, of 192 121 -> 22; 1536 rows of 8 slices 17.4 -> 14.7; 24576 rows of
+// two 22.2 both.  G = 4 from five slices on, G = 1 for fewer, where the rows
+// alone fill the card.
 template <int G>
 __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdArgs a) {
     constexpr int LPR = 16 * G;   // lanes per query
@@ -888,27 +893,39 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdArgs a) {
     auto slice_ml = [&](int s) FA2_INLINE {
         return s < nsplit ? *reinterpret_cast<const f2 *>(a.part_ml + 2 * (s * BHS + row)) : f2{-INFINITY, 0.f};
     };
-    const f2 ml0 = slice_ml(lane);
-    float M = ml0[0];
+    f4 x[4];   // the step's slices s1 + grp, s1 + G + grp, ...
+    auto load_o = [&](int s1) FA2_INLINE {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {   // (past the last slice: the last one)
+            const int64_t s = min(s1 + u * G + grp, nsplit - 1);
+            x[u] = *reinterpret_cast<const f4 *>(a.part_o + (s * BHS + row) * HD + 4 * part);
+        }
+    };
+    f2 ml = slice_ml(lane);
+    load_o(0);
+    float M = ml[0];
     for (int s0 = LPR; s0 < nsplit; s0 += LPR) M = fmaxf(M, slice_ml(s0 + lane)[0]);
 #pragma unroll
     for (int off = 1; off < LPR; off <<= 1) M = fmaxf(M, __shfl_xor(M, off));
     float lsum = 0.f;
     f4 acc = {0.f, 0.f, 0.f, 0.f};
     if (M != -INFINITY) {
-        for (int s0 = 0; s0 < nsplit; s0 += LPR) {
-            const f2 ml = s0 == 0 ? ml0 : slice_ml(s0 + lane);
-            const float w = __builtin_amdgcn_exp2f(ml[0] - M);
-            lsum += (ml[0] == -INFINITY) ? 0.f : w * ml[1];
-            const int n = min(nsplit - s0, LPR);
-#pragma unroll 4
-            for (int s = grp; s < n; s += G) {
+        float w = 0.f;
+        for (int s1 = 0; s1 < nsplit; s1 += 4 * G) {
+            if (s1 % LPR == 0) {
+                if (s1 > 0) ml = slice_ml(s1 + lane);
+                w = __builtin_amdgcn_exp2f(ml[0] - M);
+                lsum += (ml[0] == -INFINITY) ? 0.f : w * ml[1];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int s = s1 % LPR + u * G + grp;   // below LPR; past the last slice its max is -inf
                 const float ws = __shfl(w, s, LPR);
                 const bool seen = __shfl(ml[0], s, LPR) != -INFINITY;   // (a slice that saw no key is left out)
-                const f4 x = *reinterpret_cast<const f4 *>(a.part_o + ((s0 + s) * BHS + row) * HD + 4 * part);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[j] += seen ? ws * x[j] : 0.f;
+                for (int j = 0; j < 4; ++j) acc[j] += seen ? ws * x[u][j] : 0.f;
             }
+            if (s1 + 4 * G < nsplit) load_o(s1 + 4 * G);
         }
 #pragma unroll
         for (int off = 1; off < LPR; off <<= 1) lsum += __shfl_xor(lsum, off);
