@@ -275,6 +275,34 @@ def test_build_failure_path_in_fresh_process(tmp_path):
     assert out.split() == ["False", "ImportError"]
 
 
+def test_fallback_calls_trace_and_take_nested_tensors():
+    """Calls that go to SDPA stay traceable in one graph, and tensors that are no plain strided ones
+    (nested, fake, symbolic sizes) get the Python predicate's answer, not an error of the native one."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+    assert fa.is_available(), fa.build_error()
+    q = torch.randn(2, 3, 5, 64, generator=torch.Generator().manual_seed(0))
+    ref = F.scaled_dot_product_attention(q, q, q, is_causal=True)
+    for dynamic in (False, True):
+        torch._dynamo.reset()
+        traced = torch.compile(lambda x: fa.sdpa(x, x, x, is_causal=True), backend="eager", fullgraph=True,
+                               dynamic=dynamic)
+        assert torch.equal(traced(q), ref)
+    ready3 = fa.extension().ready3
+    rows = [torch.randn(3, n, 64) for n in (5, 7)]
+    nested = torch.nested.nested_tensor(rows)
+    jagged = torch.nested.nested_tensor([r.transpose(0, 1) for r in rows], layout=torch.jagged).transpose(1, 2)
+    for t in (nested, jagged):
+        assert ready3(t, t, t) == -1 and ready3(q, q, t) == -1 and not fa.can_use(t, t, t)
+    assert not fa.can_use(q, None, None)   # an ineligible q settles it
+    with FakeTensorMode():
+        t = torch.empty(2, 3, 5, 64, device="cuda", dtype=torch.float16)
+        assert ready3(t, t, t) == -1 and fa.can_use(t, t, t) and not fa.can_use(t, t, t.float())
+    seen = []
+    make_fx(lambda x: seen.append((ready3(x, x, x), fa.can_use(x, x, x))) or x + 1, tracing_mode="symbolic")(q)
+    assert seen == [(-1, False)]
+
+
 def test_eligibility_predicate_matches_reference_rules():
     """_fa_ready: fp16, 4-D, D=64, unit last stride, 32-byte base and strides."""
     class Fake:

@@ -55,10 +55,17 @@ void strides3(const torch::Tensor &t, int64_t out[3]) {
 // The module's eligibility predicate (its _fa_ready: fp16 GPU (B,H,S,64), unit
 // stride in the head dimension, 32-byte aligned base and strides) of three
 // tensors in one call: bits 0..2 are q, k, v, bit 3 is set when all have one
-// shape.  (From Python the three checks take 2.5 us, a quarter of a small
+// shape; -1, and nothing asked of their sizes, if one is no plain strided
+// tensor.  (From Python the three checks take 2.5 us, a quarter of a small
 // decode or prefill call's host time; here 0.4 us.)
 int64_t ready3(const torch::Tensor &q, const torch::Tensor &k, const torch::Tensor &v) {
     const torch::Tensor *const ts[3] = {&q, &k, &v};
+    for (const torch::Tensor *t : ts) {
+        const c10::TensorImpl *impl = t->unsafeGetTensorImpl();
+        if (!t->defined() || t->layout() != c10::kStrided || t->is_nested() || impl->is_python_dispatch() ||
+            impl->has_symbolic_sizes_strides())
+            return -1;
+    }
     int64_t bits = 0;
     for (int i = 0; i < 3; ++i) {
         const torch::Tensor &t = *ts[i];

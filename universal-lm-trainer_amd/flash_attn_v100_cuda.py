@@ -176,16 +176,33 @@ def _fa_ready(t):
             and all((s * 2) % 32 == 0 for s in t.stride()[:3]))
 
 
+def _native_bits(q, k, v):
+    """_fa_ready of q, k, v in bits 0..2 and, in bit 3, whether their shapes agree, from one native
+    call; -1 where only _fa_ready can say: tensors that are not plain ones (nested, fake, symbolic
+    sizes, subclasses), a q on the CPU, and code under torch.compile, which cannot trace the call."""
+    if _EXT is None or not q.is_cuda or torch.compiler.is_compiling():
+        return -1
+    return _EXT.ready3(q, k, v)
+
+
 def _ready_bits(q, k, v):
-    """_fa_ready of q, k, v in bits 0..2 and, in bit 3, whether their shapes agree."""
-    if _EXT is not None:
-        return _EXT.ready3(q, k, v)
-    return (_fa_ready(q) | _fa_ready(k) << 1 | _fa_ready(v) << 2) | (q.shape == k.shape == v.shape) << 3
+    """_fa_ready of q, k, v in bits 0..2."""
+    bits = _native_bits(q, k, v)
+    return bits if bits >= 0 else _fa_ready(q) | _fa_ready(k) << 1 | _fa_ready(v) << 2
+
+
+def _all_ready(q, k, v):
+    bits = _native_bits(q, k, v)
+    return bits & 7 == 7 if bits >= 0 else _fa_ready(q) and _fa_ready(k) and _fa_ready(v)
 
 
 def can_use(q, k, v):
     """Whether the tensors can go to the kernel directly (reference :105-108)."""
-    return _ready_bits(q, k, v) == 15
+    bits = _native_bits(q, k, v)
+    if bits >= 0:
+        return bits == 15
+    return (_fa_ready(q) and _fa_ready(k) and _fa_ready(v)
+            and q.shape == k.shape == v.shape)
 
 
 class _RopeV100Cuda(torch.autograd.Function):
@@ -252,7 +269,7 @@ def _needs_grad(*ts):
 
 def _kv_ready(q, k, v):
     """fp16 (B,H,S_q,64) queries against (B,H,S_k,64) keys/values, kernel-aligned."""
-    return (_ready_bits(q, k, v) & 7 == 7 and k.shape == v.shape
+    return (_all_ready(q, k, v) and k.shape == v.shape
             and k.shape[:2] == q.shape[:2] and k.size(2) >= 1)
 
 
