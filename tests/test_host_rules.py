@@ -1,0 +1,53 @@
+"""Rules of the launchers that no result shows (which variant a call takes), compiled for the host."""
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "universal-lm-trainer_amd", "csrc")
+HIPCC = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "bin", "hipcc")
+
+
+@pytest.fixture(scope="module")
+def evaluate(tmp_path_factory):
+    """evaluate(expressions) -> their values as integers, with namespace fa2 open and `args(...)` at hand."""
+    def run(expressions):
+        d = tmp_path_factory.mktemp("rules")
+        src = d / "rules.cpp"
+        src.write_text('#include "%s/fa2_kernels.h"\n#include <cstdio>\nusing namespace fa2;\n' % CSRC + """
+static FwdArgs args(int B, int H, int Sk, int coff, int64_t sb, int64_t sh, int64_t ss, bool v_only = false) {
+    FwdArgs a = {};
+    a.B = B; a.H = H; a.S = 1; a.Sk = Sk; a.coff = coff;
+    a.vsb = sb; a.vsh = sh; a.vss = ss;
+    a.ksb = v_only ? (int64_t)H * Sk * 64 : sb; a.ksh = v_only ? (int64_t)Sk * 64 : sh; a.kss = v_only ? 64 : ss;
+    return a;
+}
+int main() {
+""" + "\n".join(f'printf("%lld\\n", (long long)({e}));' for e in expressions) + "\n}\n")
+        exe = d / "rules"
+        subprocess.run([HIPCC, "-x", "hip", "--offload-host-only", "-std=c++17", str(src), "-o", str(exe)], check=True,
+                       capture_output=True)
+        return [int(x) for x in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()]
+    return run
+
+
+def test_decode_streams_large_caches_read_once(evaluate):
+    """80 MiB of K and V is B*H*keys = 327680."""
+    n = 16384
+    dense = (12 * n * 64, n * 64, 64)
+    cases = [
+        (1, "args(8, 12, %d, %d, %d, %d, %d), true" % (n, n - 1, *dense)),
+        (1, "args(8, 12, %d, %d, %d, %d, %d), false" % (n, 0, *dense)),
+        (0, "args(8, 12, %d, %d, %d, %d, %d), true" % (n, 3000, *dense)),        # 3001 keys seen
+        (0, "args(8, 12, %d, %d, %d, %d, %d), true" % (n, -1, *dense)),
+        (1, "args(8, 12, %d, %d, %d, 64, 768), true" % (n, n - 1, n * 768)),     # [B, S, H, D]
+        (1, "args(8, 12, %d, %d, %d, %d, 64), true" % (n, n - 1, 12 * (n + 128) * 64, (n + 128) * 64)),   # spare keys
+        (0, "args(8, 12, %d, %d, %d, 0, 64), true" % (n, n - 1, n * 64)),        # one head for all
+        (0, "args(8, 12, %d, %d, 0, %d, 64), true" % (n, n - 1, n * 64)),        # one batch for all
+        (0, "args(8, 12, %d, %d, %d, 0, 64, true), true" % (n, n - 1, n * 64)),  # V alone
+        (0, "args(8, 12, %d, %d, %d, %d, 8), true" % (n, n - 1, 12 * n * 8, n * 8)),   # rows overlap
+        (1, "args(1, 1, 400000, 399999, 0, 0, 64), true"),                       # strides of single heads don't count
+        (0, "args(1, 20, 16384, 16383, %d, %d, 64), true" % (20 * n * 64, n * 64)),    # exactly 80 MiB
+    ]
+    got = evaluate(["decode_streams(%s)" % c for _, c in cases])
+    assert got == [e for e, _ in cases]

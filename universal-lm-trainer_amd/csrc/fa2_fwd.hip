@@ -966,14 +966,8 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdArgs a) {
 // waves per workgroup (four: 5-30% slower where a head has one workgroup,
 // sixteen: equal there, slower with many heads).
 //
-// STREAM: K and V by nontemporal loads, for a cache that takes more than a
-// third of the 256 MB Infinity Cache (DEC_STREAM_BYTES) and will not be there
-// at the next token: 70 -> 58.7 us at 403 MB (B*H = 96, Sk = 16384; 6.9 TB/s),
-// 19.8 -> 18.9 us at 101 MB.  Smaller caches can stay there and plain loads
-// are then as fast or faster (74 MB: 14.2 us against 14.7, 12.6 MB in one slice
-// 14.1 against 20.1).
+// STREAM: K and V by nontemporal loads (decode_streams).
 constexpr int DEC_NW = 8;
-constexpr int64_t DEC_STREAM_BYTES = 80 << 20;
 
 // Sum over the 8 lanes of each aligned group of 8, returned to all of them:
 // DPP quad_perm [1,0,3,2] and [2,3,0,1] (partners xor 1, xor 2), then
@@ -1235,8 +1229,7 @@ static hipError_t launch_decode(const FwdArgs &a_in, hipStream_t st) {
 }
 
 hipError_t launch_fwd_decode(const FwdArgs &a, bool causal, hipStream_t st) {
-    const int64_t keys = causal ? std::max<int64_t>(0, std::min<int64_t>(a.Sk, (int64_t)a.coff + 1)) : a.Sk;   // read
-    const bool stream = (int64_t)a.B * a.H * keys * HD * 2 * (int64_t)sizeof(_Float16) > DEC_STREAM_BYTES;
+    const bool stream = decode_streams(a, causal);
     const hipError_t e = causal ? (stream ? launch_decode<true, true>(a, st) : launch_decode<true, false>(a, st))
                                 : (stream ? launch_decode<false, true>(a, st) : launch_decode<false, false>(a, st));
     return (e != hipSuccess || a.nsplit <= 1) ? e : launch_combine(a, st);

@@ -115,6 +115,30 @@ inline int query_block_base(bool causal, int S, int qwg, int64_t wgs, int64_t sl
 // 2^24 - 1 heads of one block keep below.
 inline int grid_heads(int64_t bh) { return (int)(bh >= 128 && bh < (1 << 20) ? (bh + 7) & ~(int64_t)7 : bh); }
 
+// Whether a [B, H, keys, 64] view (strides in elements, not negative) holds
+// that many elements: false for one expanded over batches, heads or keys
+// (stride 0) and for overlapping rows.
+inline bool view_is_dense(int B, int H, int64_t keys, int64_t sb, int64_t sh, int64_t ss) {
+    if ((B > 1 && sb == 0) || (H > 1 && sh == 0) || (keys > 1 && ss == 0)) return false;
+    return (B - 1) * sb + (H - 1) * sh + (keys - 1) * ss + 64 >= (int64_t)B * H * keys * 64;
+}
+
+// Decode reads K and V by nontemporal loads when they take more than 80 MiB, a
+// third of the 256 MB Infinity Cache: 70 -> 58.7 us at 403 MB (B*H = 96,
+// Sk = 16384; 6.9 TB/s), 19.8 -> 18.9 us at 101 MB.  Smaller caches can stay
+// there from one call to the next and plain loads are then as fast or faster
+// (74 MB, called again and again: 14.2 us against 14.7; 12.6 MB in one slice 14.1
+// against 20.1).  A cache whose heads or batches share their rows is read many
+// times and keeps plain loads: B=64 H=16 Sk=4096 expanded over the heads 80 us
+// against 125, B=8 H=12 Sk=16384 over the batches 29 against 46.
+inline bool decode_streams(const FwdArgs &a, bool causal) {
+    constexpr int64_t BYTES = 80 << 20;
+    int64_t keys = a.Sk;
+    if (causal && (int64_t)a.coff + 1 < keys) keys = a.coff + 1 > 0 ? a.coff + 1 : 0;   // the keys read
+    return (int64_t)a.B * a.H * keys * 64 * 2 * (int64_t)sizeof(_Float16) > BYTES &&
+           view_is_dense(a.B, a.H, keys, a.ksb, a.ksh, a.kss) && view_is_dense(a.B, a.H, keys, a.vsb, a.vsh, a.vss);
+}
+
 // Compute units of the current device (cached per device; 256 on MI355X).
 // Launchers use it to size grids against the slots of two workgroups per CU.
 int device_cus();
