@@ -54,6 +54,21 @@ def split_inputs(H, Sq, Sk):
     return q, k, v
 
 
+@pytest.mark.parametrize("Sk", [1, 64, 65, 255, 256, 257, 320])
+def test_decode_wave_counts(fa, Sk):
+    """Slices of at most 256 keys take four waves, longer ones eight: the same bits as from a longer
+    cache whose further keys are hidden (eight waves)."""
+    print(f"case decode waves Sk={Sk}", flush=True)
+    ext = fa.extension()
+    q, k, v = split_inputs(3, 1, 600)
+    o, lse = ext.fa_fwd_kv(q, k[:, :, :Sk], v[:, :, :Sk], True, 0.125, Sk - 1, 1)
+    o8, lse8 = ext.fa_fwd_kv(q, k, v, True, 0.125, Sk - 1, 1)
+    assert torch.equal(o, o8) and torch.equal(lse, lse8)
+    ro, rl = reference(q, k, v, Sk)
+    assert (o.float() - ro).abs().max().item() <= O_TOL * max(1.0, ro.abs().max().item() / 2)
+    assert (lse - rl).abs().max().item() <= 1e-3
+
+
 @pytest.mark.parametrize("Sq", [1, 5])
 @pytest.mark.parametrize("lo", [1, 65, 129])
 def test_merge_every_slice_count(fa, Sq, lo):

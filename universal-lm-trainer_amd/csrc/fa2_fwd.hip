@@ -962,12 +962,10 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdArgs a) {
 // Bound by what one CU can keep in flight (57 GB/s per CU at most, whatever
 // the number of waves) and, with every CU at work, by HBM.  A wave holds one
 // block's rows in registers: the next block's K rows are requested as soon as
-// the scores have consumed this one's, its V rows after the P V sums.  Eight
-// waves per workgroup (four: 5-30% slower where a head has one workgroup,
-// sixteen: equal there, slower with many heads).
+// the scores have consumed this one's, its V rows after the P V sums.  DEC_NW
+// waves per workgroup (decode_waves).
 //
 // STREAM: K and V by nontemporal loads (decode_streams).
-constexpr int DEC_NW = 8;
 
 // Sum over the 8 lanes of each aligned group of 8, returned to all of them:
 // DPP quad_perm [1,0,3,2] and [2,3,0,1] (partners xor 1, xor 2), then
@@ -989,7 +987,7 @@ __device__ __forceinline__ void merge_state(float &m, float &l, f8 &acc, float m
     m = mx;
 }
 
-template <bool CAUSAL, bool STREAM>
+template <bool CAUSAL, bool STREAM, int DEC_NW>
 __global__ __launch_bounds__(DEC_NW * 64) void decode_kernel(const FwdArgs a) {
     __shared__ float sm[DEC_NW][HD + 2];   // per wave: O accumulator, max, sum
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 3, c8 = lane & 7;
@@ -1212,7 +1210,7 @@ static hipError_t launch_combine(const FwdArgs &a, hipStream_t st) {
     return hipGetLastError();
 }
 
-template <bool CAUSAL, bool STREAM>
+template <bool CAUSAL, bool STREAM, int DEC_NW>
 static hipError_t launch_decode(const FwdArgs &a_in, hipStream_t st) {
     FwdArgs a = a_in;
     // 2^22 workgroups per launch at most: the launch limit of 2^32 threads is
@@ -1220,12 +1218,17 @@ static hipError_t launch_decode(const FwdArgs &a_in, hipStream_t st) {
     const int64_t wgs = (int64_t)a.B * a.H * a.nsplit, per = 1 << 22;
     for (int64_t w = 0; w < wgs; w += per) {
         a.wg0 = (int)w;
-        hipLaunchKernelGGL((decode_kernel<CAUSAL, STREAM>), dim3((unsigned)std::min(per, wgs - w)), dim3(DEC_NW * 64),
+        hipLaunchKernelGGL((decode_kernel<CAUSAL, STREAM, DEC_NW>), dim3((unsigned)std::min(per, wgs - w)), dim3(DEC_NW * 64),
                            0, st, a);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
+}
+
+template <bool CAUSAL, bool STREAM>
+static hipError_t launch_decode(const FwdArgs &a, hipStream_t st) {
+    return decode_waves(a) == 4 ? launch_decode<CAUSAL, STREAM, 4>(a, st) : launch_decode<CAUSAL, STREAM, 8>(a, st);
 }
 
 hipError_t launch_fwd_decode(const FwdArgs &a, bool causal, hipStream_t st) {

@@ -139,6 +139,14 @@ inline bool decode_streams(const FwdArgs &a, bool causal) {
            view_is_dense(a.B, a.H, keys, a.ksb, a.ksh, a.kss) && view_is_dense(a.B, a.H, keys, a.vsb, a.vsh, a.vss);
 }
 
+// Waves of a decode workgroup: eight, or four for slices of at most 256 keys,
+// which give each of four waves one 64-key block (and the same sums).  Four are
+// 5-30% slower on longer slices where a head has one workgroup, sixteen equal
+// there and slower with many heads; eight, half of them idle, take the slots of
+// workgroups that have not started (B*H = 768: 64 keys 5.5 us against 3.8, 200
+// keys 8.0 against 7.2).
+inline int decode_waves(const FwdArgs &a) { return a.split_keys <= 256 ? 4 : 8; }
+
 // Compute units of the current device (cached per device; 256 on MI355X).
 // Launchers use it to size grids against the slots of two workgroups per CU.
 int device_cus();
