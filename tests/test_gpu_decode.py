@@ -104,6 +104,17 @@ def test_merge_of_automatic_slices(fa, H, Sq, Sk, slices):
     assert (o.float() - ro).abs().max().item() <= O_TOL
 
 
+@pytest.mark.parametrize("H,Sk,slices", [(12, 1535, 1), (12, 1536, 6), (79, 1536, 3), (80, 2047, 1), (80, 2048, 3),
+                                         (96, 2047, 1), (128, 1536, 1), (128, 2048, 2), (129, 4096, 1)])
+def test_decode_automatic_slices(fa, H, Sk, slices):
+    """Both sides of the slice rule's lines: the same bits as with the count given."""
+    print(f"case decode slice rule H={H} Sk={Sk}", flush=True)
+    ext = fa.extension()
+    q, k, v = split_inputs(H, 1, Sk)
+    for a, b in zip(ext.fa_fwd_kv(q, k, v, True, 0.125, Sk - 1, 0), ext.fa_fwd_kv(q, k, v, True, 0.125, Sk - 1, slices)):
+        assert torch.equal(a, b)
+
+
 def test_decode_merge_edges(fa):
     """The merge of slices gives NaN where a slice's softmax met an infinite score (inf - inf), and a
     query that sees no key gives O = 0 and LSE = -inf with one slice and with several."""
