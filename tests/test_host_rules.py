@@ -1,11 +1,16 @@
 """Rules of the launchers that no result shows (which variant a call takes), compiled for the host."""
+import glob
 import os
+import shutil
 import subprocess
 
 import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "universal-lm-trainer_amd", "csrc")
-HIPCC = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "bin", "hipcc")
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+HIPCC = os.path.join(ROCM, "bin", "hipcc")
+OBJDUMP = os.path.join(ROCM, "llvm", "bin", "llvm-objdump")
+LIB = os.path.join(os.path.dirname(CSRC), "lib", "libfa2_mi355x.so")
 
 
 @pytest.fixture(scope="module")
@@ -51,3 +56,18 @@ def test_decode_streams_large_caches_read_once(evaluate):
     ]
     got = evaluate(["decode_streams(%s)" % c for _, c in cases])
     assert got == [e for e, _ in cases]
+
+
+def test_kernels_access_memory_by_address_space(tmp_path):
+    """No flat loads or stores (they count as LDS accesses too, and every wait for an LDS read would wait
+    for them) and no scratch in the kernels as built."""
+    shutil.copy(LIB, tmp_path / "lib.so")
+    subprocess.run([OBJDUMP, "--offloading", "lib.so"], cwd=tmp_path, check=True, capture_output=True)
+    objects = glob.glob(str(tmp_path / "lib.so.*gfx950"))
+    assert len(objects) >= 3
+    count = {"flat_": 0, "scratch_": 0, "global_": 0}
+    for o in objects:
+        for line in subprocess.run([OBJDUMP, "-d", o], check=True, capture_output=True, text=True).stdout.splitlines():
+            for kind in count:
+                count[kind] += line.strip().startswith(kind)
+    assert count["global_"] > 100 and count["flat_"] == 0 and count["scratch_"] == 0, count

@@ -617,16 +617,6 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
             else if (n == 1) vm_wait<2 * TPW>();
             else vm_wait<4 * TPW>();
         };
-#ifndef FA2_FWD_STORE_SLACK
-#define FA2_FWD_STORE_SLACK 0
-#endif
-        // The same with the previous tile's keep-word store (issued after
-        // every transfer being waited for) allowed to stay in flight.
-        auto wait_tiles_st = [&](int n) FA2_INLINE {
-            if (n <= 0) vm_wait<1>();
-            else if (n == 1) vm_wait<2 * TPW + 1>();
-            else vm_wait<4 * TPW + 1>();
-        };
         if (NSK - 1 < ntiles) issue_next();   // the last stage's tile (the prologue sent the others)
         wait_tiles(min(NSK - 1, ntiles - 1));
         lds_barrier();                         // tile 0 landed for every wave
@@ -643,6 +633,9 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
         // next tile's transfers; without either, and with the loop unrolled
         // as below, the forward with words goes from 238 to 223.5 us at B=15
         // H=12 S=2050 and from 139.6 to 135 at B=32 S=1024.)
+        // (An address formed from an integer names no address space: said here,
+        // or the store is a flat one, which the next tile's LDS reads wait for.)
+        typedef __attribute__((address_space(1))) uint32_t global_u32;
         uint64_t dm = DMASK ? (uint64_t)(uintptr_t)(a.drop_mask + dmask_word(CAUSAL, bh, S, 0, 0, qw0)) : 0u;
         int dn = DMASK ? dmask_run(CAUSAL, S, 0) : 0;
         for (int t0 = 0; t0 < ntiles; t0 += NSK) {
@@ -653,10 +646,7 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
                 uint32_t w = 0;
                 if (t <= tlast) w = inorder_tile(t, ph, s, p);
                 if (t + 1 < ntiles) {
-                    if (DMASK && FA2_FWD_STORE_SLACK && t >= 1 && t - 1 <= tlast)
-                        wait_tiles_st(min(NSK - 2, ntiles - 2 - t));
-                    else
-                        wait_tiles(min(NSK - 2, ntiles - 2 - t));   // tile t+1 landed
+                    wait_tiles(min(NSK - 2, ntiles - 2 - t));   // tile t+1 landed
                     lds_barrier();
                     if (t + NSK < ntiles) issue_next();
                 }
@@ -664,7 +654,7 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
                     if (t <= tlast) {
                         const int ln = fresh_lane(), r = ln & 31;   // query qw0 + r (QB == 1)
                         if (qw0 + r < S)
-                            *reinterpret_cast<uint32_t *>(dm + 4u * (mul_u24((uint32_t)dn, (uint32_t)ln >> 5) + (uint32_t)r)) = w;
+                            *reinterpret_cast<global_u32 *>(dm + 4u * (mul_u24((uint32_t)dn, (uint32_t)ln >> 5) + (uint32_t)r)) = w;
                     }
                     // Next tile's run; a 128-key block's runs start 128 queries later.
                     const bool next_block = CAUSAL && (t & 1);
