@@ -129,6 +129,10 @@ __global__ __launch_bounds__(256, NARROW ? DQ_NARROW_WAVES : 2) void bwd_dq_pipe
     const int BH = a.B * a.H;
     const int nqblk = (S + QWG - 1) / QWG;
     int qslot, bh;
+    touch_arg(a.q);
+    touch_arg(a.qsb);
+    touch_arg(a.vsb);
+    touch_arg(a.doss);
     query_block_order(blockIdx.x, a.bhp, nqblk, a.hgroup, qslot, bh);
     if (bh >= BH) return;
     const int qblk = nqblk - 1 - qslot;   // heaviest (last) query blocks first
@@ -942,6 +946,11 @@ __global__ __launch_bounds__(256, 2) void bwd_dkv_pipe_kernel(const BwdArgs a) {
     const bool pair = CAUSAL && !DROPOUT && a.dkv_pair;
     const int nwg_head = pair ? (nkb + 1) / 2 : nkb;   // workgroups per head
     const int L = blockIdx.x;
+    touch_arg(a.q);
+    touch_arg(a.qsb);
+    touch_arg(a.vsb);
+    touch_arg(a.doss);
+    touch_arg(a.bhp);
     int j, bh;
     if (pair && (BH & 7) == 0) {
         const int xcd = L & 7, i = L >> 3;
