@@ -58,6 +58,21 @@ def test_decode_streams_large_caches_read_once(evaluate):
     assert got == [e for e, _ in cases]
 
 
+def test_head_groups(evaluate):
+    """Multiples of eight heads in groups as ever; rounded head numbers under the causal mask only where
+    the last, partial group does not set the time (768 dQ workgroups resident)."""
+    cases = [
+        (1, "fwd_groups(8, true, 8)"), (1, "fwd_groups(136, true, 8)"), (0, "fwd_groups(127, false, 8)"),
+        (0, "fwd_groups(132, true, 8)"), (1, "fwd_groups(132, false, 8)"), (0, "fwd_groups(372, true, 5)"),
+        (1, "fwd_groups(372, true, 4)"), (0, "fwd_groups(428, true, 8)"), (1, "fwd_groups(444, true, 8)"),
+        (0, "fwd_groups((1 << 20) + 1, true, 1)"),
+        (1, "dq_groups(128, true, 512, 768)"), (0, "dq_groups(132, true, 544, 768)"),
+        (1, "dq_groups(132, false, 544, 768)"), (0, "dq_groups(188, true, 768, 768)"),
+        (1, "dq_groups(196, true, 800, 768)"), (0, "dq_groups(100, true, 800, 768)"),
+    ]
+    assert evaluate([c for _, c in cases]) == [e for e, _ in cases]
+
+
 def test_kernels_access_memory_by_address_space(tmp_path):
     """No flat loads or stores (they count as LDS accesses too, and every wait for an LDS read would wait
     for them) and no scratch in the kernels as built."""

@@ -1011,10 +1011,11 @@ hipError_t launch_bwd_delta(const BwdArgs &a, hipStream_t st) {
 template <bool NARROW>
 static void launch_dq_t(const BwdArgs &a_in, bool causal, bool dropout, hipStream_t st) {
     BwdArgs a = a_in;
-    a.hgroup = !dropout && a.bhp % 8 == 0 && a.S <= FA2_DQ_GROUP_MAX_S ? 16 : 0;
     const int qwg = NARROW && !(dropout && a.drop_mask != nullptr) ? DQ_NW * 32 : DQ_QWG;
     const dim3 grid((unsigned)((a.S + qwg - 1) / qwg * a.bhp)), block(256);
-    a.qbase = query_block_base(causal, a.S, qwg, grid.x, (int64_t)(qwg == DQ_QWG ? 2 : DQ_NARROW_WAVES) * device_cus());
+    const int64_t slots = (int64_t)(qwg == DQ_QWG ? 2 : DQ_NARROW_WAVES) * device_cus();
+    a.hgroup = !dropout && a.S <= FA2_DQ_GROUP_MAX_S && dq_groups((int64_t)a.B * a.H, causal, grid.x, slots) ? 16 : 0;
+    a.qbase = query_block_base(causal, a.S, qwg, grid.x, slots);
     const bool dmask = dropout && a.drop_mask != nullptr;
     if (causal) {
         if (dmask)

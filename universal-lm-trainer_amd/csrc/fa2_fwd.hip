@@ -1133,7 +1133,9 @@ void launch_fwd_t(const FwdArgs &a_in, bool causal, bool dropout, hipStream_t st
     // was 5-16% slower there).
     const int64_t narrow_wgs = (int64_t)((a.S + qwg_of(1) - 1) / qwg_of(1)) * a.B * a.H;
     if (!SPLIT && FA2_FWD_NARROW && narrow_wgs >= (int64_t)NARROW_WAVES * device_cus()) {
-        if (!dropout && a.bhp % 8 == 0 && a.S <= FA2_FWD_GROUP_MAX_S) a.hgroup = 16;
+        if (!dropout && a.S <= FA2_FWD_GROUP_MAX_S &&
+            fwd_groups((int64_t)a.B * a.H, causal, (a.S + qwg_of(1) - 1) / qwg_of(1)))
+            a.hgroup = 16;
         a.qbase = query_block_base(causal, a.S, qwg_of(1), narrow_wgs, (int64_t)NARROW_WAVES * device_cus());
         if (causal) {
             if (dmask) launch_narrow<true, true, true>(a, st);
