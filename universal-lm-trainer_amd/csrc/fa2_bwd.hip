@@ -946,11 +946,13 @@ __global__ __launch_bounds__(256, 2) void bwd_dkv_pipe_kernel(const BwdArgs a) {
     const bool pair = CAUSAL && !DROPOUT && a.dkv_pair;
     const int nwg_head = pair ? (nkb + 1) / 2 : nkb;   // workgroups per head
     const int L = blockIdx.x;
-    touch_arg(a.q);
-    touch_arg(a.qsb);
-    touch_arg(a.vsb);
-    touch_arg(a.doss);
-    touch_arg(a.bhp);
+    if (!DROPOUT) {
+        touch_arg(a.q);
+        touch_arg(a.qsb);
+        touch_arg(a.vsb);
+        touch_arg(a.doss);
+        touch_arg(a.bhp);
+    }
     int j, bh;
     if (pair && (BH & 7) == 0) {
         const int xcd = L & 7, i = L >> 3;

@@ -451,7 +451,9 @@ __device__ __forceinline__ int64_t dmask_word(bool causal, int bh, int S, int t6
 // arguments' own loads behind that exit, where they would start from memory only
 // after the head's divisions.  (S = 64, 8 heads, against exit and no touch:
 // forward 4.60 -> 4.17 us, dQ pass 5.50 -> 5.34, dK/dV pass 5.42 -> 5.20; 4.35,
-// 5.30 and 5.35 without the exit either.  S = 4096, 96 heads: equal.)
+// 5.30 and 5.35 without the exit either.  S = 4096, 96 heads: equal.)  Left out
+// where the tile loop as compiled takes longer for it: 4% in the forward without
+// the mask (its first line only), 1% in the dK/dV pass with dropout.
 __device__ __forceinline__ void touch_arg(int64_t v) { asm volatile("" : : "s"((uint32_t)v)); }
 __device__ __forceinline__ void touch_arg(const void *p) { touch_arg((int64_t)(uintptr_t)p); }
 

@@ -133,7 +133,7 @@ __global__ __launch_bounds__(NW * 64, NARROW ? NARROW_WAVES : 8 / NW) void fwd_k
         ks = rem / BH;
         bh = rem - ks * BH;
     } else {
-        touch_arg(a.q);
+        if (CAUSAL) touch_arg(a.q);
         touch_arg(a.ksb);
         query_block_order(L, a.bhp, nqblk, a.hgroup, qslot, bh);
         if (bh >= BH) return;
