@@ -65,7 +65,8 @@ def test_head_groups(evaluate):
         (1, "fwd_groups(8, true, 8)"), (1, "fwd_groups(136, true, 8)"), (0, "fwd_groups(127, false, 8)"),
         (0, "fwd_groups(132, true, 8)"), (1, "fwd_groups(132, false, 8)"), (0, "fwd_groups(372, true, 5)"),
         (1, "fwd_groups(372, true, 4)"), (0, "fwd_groups(428, true, 8)"), (1, "fwd_groups(444, true, 8)"),
-        (0, "fwd_groups((1 << 20) + 1, true, 1)"),
+        (0, "fwd_groups((1 << 20) + 1, true, 2)"), (0, "fwd_groups(1024, true, 1)"), (1, "fwd_groups(1024, true, 2)"),
+        (0, "dq_groups(1024, true, 1024, 768)"), (0, "dq_groups(1500, true, 1504, 768)"),
         (1, "dq_groups(128, true, 512, 768)"), (0, "dq_groups(132, true, 544, 768)"),
         (1, "dq_groups(132, false, 544, 768)"), (0, "dq_groups(188, true, 768, 768)"),
         (1, "dq_groups(196, true, 800, 768)"), (0, "dq_groups(100, true, 800, 768)"),

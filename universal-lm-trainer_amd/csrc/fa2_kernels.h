@@ -112,27 +112,29 @@ inline int query_block_base(bool causal, int S, int qwg, int64_t wgs, int64_t sl
 // on: with fewer, the XCDs with one head more set the time (108 heads at
 // S = 1500: dQ pass 67 -> 71 us); with 129, 17 heads on one XCD and 16 on the
 // others, the shared tiles outweigh it (S = 1050 forward 33.0 -> 29.6, backward
-// 100.3 -> 97.3; S = 2050 99.0 -> 86.6, 285 -> 278).  Not from 2^20 heads on: the rounding gains
-// nothing there and could reach the launch limit of 2^32 threads, which
-// 2^24 - 1 heads of one block keep below.
+// 100.3 -> 97.3; S = 2050 99.0 -> 86.6, 285 -> 278).  Not from 2^20 heads on:
+// the rounding gains nothing there and could reach the launch limit of 2^32
+// threads, which 2^24 - 1 heads of one block keep below.
 inline int grid_heads(int64_t bh) { return (int)(bh >= 128 && bh < (1 << 20) ? (bh + 7) & ~(int64_t)7 : bh); }
 
 // Whether the forward (`nq` query blocks a head) and the dQ pass (`wgs`
 // workgroups in all, `slots` of them resident) take an XCD's heads in groups
 // (query_block_order), where their lengths make groups pay.  Groups need whole
-// XCDs of heads.  Rounded head numbers (grid_heads) leave a last group of any
-// size, whose heaviest blocks come late in the grid, and under the causal mask
-// that can cost more than the shared tiles save: in the dQ pass while the grid
-// is resident at once (H = 12, B=11 S=512 21.7 us in groups, 17.8 plain; 188 heads
-// 23.7, 21.5; B=17 24.1, 25.2), in the forward of five blocks and more
-// up to 432 heads (B=11 S=1024 37.0 us in groups, 30.7 plain; B=25 S=640 32.9,
-// 30.0; B=37 S=1024 87.8, 89.5).  With up to four blocks neither is the faster
-// throughout (S = 512: B=31 26.4, 27.3; B=33 30.1, 28.5).
+// XCDs of heads, and with one block a head they are the plain order at the price
+// of another division (B=125 H=12 S=19 forward 8.81 us, 8.52 plain).  Rounded
+// head numbers (grid_heads) leave a last group of any size, whose heaviest blocks
+// come late in the grid, and under the causal mask that can cost more than the
+// shared tiles save: in the dQ pass while the grid is resident at once (H = 12,
+// B=11 S=512 21.7 us in groups, 17.8 plain; 188 heads 23.7, 21.5; B=17 24.1,
+// 25.2), in the forward of five blocks and more up to 432 heads (B=11 S=1024
+// 37.0 us in groups, 30.7 plain; B=25 S=640 32.9, 30.0; B=37 S=1024 87.8, 89.5).
+// With up to four blocks neither is the faster throughout (S = 512: B=31 26.4,
+// 27.3; B=33 30.1, 28.5).
 inline bool fwd_groups(int64_t bh, bool causal, int nq) {
-    return grid_heads(bh) % 8 == 0 && (bh % 8 == 0 || !causal || nq <= 4 || bh > 432);
+    return nq > 1 && grid_heads(bh) % 8 == 0 && (bh % 8 == 0 || !causal || nq <= 4 || bh > 432);
 }
 inline bool dq_groups(int64_t bh, bool causal, int64_t wgs, int64_t slots) {
-    return grid_heads(bh) % 8 == 0 && (bh % 8 == 0 || !causal || wgs > slots);
+    return wgs > grid_heads(bh) && grid_heads(bh) % 8 == 0 && (bh % 8 == 0 || !causal || wgs > slots);
 }
 
 // Whether a [B, H, keys, 64] view (strides in elements, not negative) holds
