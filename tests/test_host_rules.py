@@ -15,7 +15,7 @@ LIB = os.path.join(os.path.dirname(CSRC), "lib", "libfa2_mi355x.so")
 
 @pytest.fixture(scope="module")
 def evaluate(tmp_path_factory):
-    """evaluate(expressions) -> their values as integers, with namespace fa2 open and `args(...)` at hand."""
+    """evaluate(expressions) -> their values as integers, with namespace fa2 open and `args` / `rope_args` at hand."""
     def run(expressions):
         d = tmp_path_factory.mktemp("rules")
         src = d / "rules.cpp"
@@ -25,6 +25,12 @@ static FwdArgs args(int B, int H, int Sk, int coff, int64_t sb, int64_t sh, int6
     a.B = B; a.H = H; a.S = 1; a.Sk = Sk; a.coff = coff;
     a.vsb = sb; a.vsh = sh; a.vss = ss;
     a.ksb = v_only ? (int64_t)H * Sk * 64 : sb; a.ksh = v_only ? (int64_t)Sk * 64 : sh; a.kss = v_only ? 64 : ss;
+    return a;
+}
+static RopeArgs rope_args(int B, int H, int S, int64_t k_head) {
+    RopeArgs a = {};
+    a.B = B; a.H = H; a.S = S;
+    a.qsb = a.ksb = (int64_t)S * 3 * H * 64; a.qss = a.kss = 3 * H * 64; a.qsh = 64; a.ksh = k_head;
     return a;
 }
 int main() {
@@ -56,6 +62,15 @@ def test_decode_streams_large_caches_read_once(evaluate):
     ]
     got = evaluate(["decode_streams(%s)" % c for _, c in cases])
     assert got == [e for e, _ in cases]
+
+
+def test_rope_streams_large_tensors(evaluate):
+    """88 MiB of q and k is B*H*S = 360448; a k expanded over the heads is read from the caches."""
+    cases = [
+        (1, "rope_args(8, 12, 4096, 64)"), (0, "rope_args(8, 12, 2048, 64)"), (0, "rope_args(8, 11, 4096, 64)"),
+        (1, "rope_args(8, 11, 4097, 64)"), (0, "rope_args(16, 12, 4096, 0)"),
+    ]
+    assert evaluate(["rope_streams(%s)" % c for _, c in cases]) == [e for e, _ in cases]
 
 
 def test_head_groups(evaluate):

@@ -145,6 +145,21 @@ inline bool view_is_dense(int B, int H, int64_t keys, int64_t sb, int64_t sh, in
     return (B - 1) * sb + (H - 1) * sh + (keys - 1) * ss + 64 >= (int64_t)B * H * keys * 64;
 }
 
+// RoPE reads q and k by nontemporal loads when they take more than 88 MiB
+// together: each row is read once, in whole 128-byte lines, and leaves the caches
+// to the outputs, which attention reads next.  Smaller ones are still in the
+// Infinity Cache from what made them, and plain loads find them there.  H = 12,
+// S = 2048, plain -> nontemporal: the kernel on the same tensors again and again
+// B=4 (24 MiB) 8.8 -> 10.1 us, B=14 (84 MiB) 26.2 -> 29.2, B=16 S=4096 (192 MiB)
+// 70.7 -> 59.5; a copy that makes qkv, the rope and the attention forward
+// together B=4 60.6 -> 60.9, B=14 181.5 -> 182.0, B=16 (96 MiB) 211.5 -> 206.1,
+// B=16 S=4096 630 -> 626; attention backward, rope and a reader B=14 410.7 ->
+// 412.3, B=16 S=4096 1554 -> 1543.
+inline bool rope_streams(const RopeArgs &a) {
+    return (int64_t)a.B * a.H * a.S * 64 * 2 * (int64_t)sizeof(_Float16) > (int64_t)88 << 20 &&
+           view_is_dense(a.B, a.H, a.S, a.qsb, a.qsh, a.qss) && view_is_dense(a.B, a.H, a.S, a.ksb, a.ksh, a.kss);
+}
+
 // Decode reads K and V by nontemporal loads when they take more than 80 MiB, a
 // third of the 256 MB Infinity Cache: 70 -> 58.7 us at 403 MB (B*H = 96,
 // Sk = 16384; 6.9 TB/s), 19.8 -> 18.9 us at 101 MB.  Smaller caches can stay

@@ -55,7 +55,8 @@ __device__ __forceinline__ h8 swap4(h8 v) {   // the value held by lane ^ 4
     return __builtin_bit_cast(h8, w);
 }
 
-template <bool BACKWARD>
+// STREAM: q and k by nontemporal loads (rope_streams).
+template <bool BACKWARD, bool STREAM>
 __global__ __launch_bounds__(256) void rope_vec_kernel(const RopeArgs a) {
     // B*H*S < 2^31 (host check): 32-bit row arithmetic
     const uint32_t H = (uint32_t)a.H, S = (uint32_t)a.S;
@@ -72,13 +73,10 @@ __global__ __launch_bounds__(256) void rope_vec_kernel(const RopeArgs a) {
     // backward: sin at the partner index, partner sign +1 for d < 32.
     const f8v snv = *reinterpret_cast<const f8v_a16 *>(snr + 8 * (BACKWARD ? (j ^ 4) : j));
     const float sg = (j < 4) == BACKWARD ? 1.f : -1.f;
-    // Nontemporal: each row is read once, in whole 128-byte lines, and leaves
-    // the caches to the outputs, which attention reads next (B=8 H=12 S=4096:
-    // kernel 37.9 -> 32.5 us; a producer of qkv, the rope and a reader of its
-    // outputs 115 -> 104 us together, at B=4 55 -> 53; streaming the stores
-    // too, or two rows per group of lanes: 35 and 36 us).
-    const h8 xq = __builtin_nontemporal_load(reinterpret_cast<const h8 *>(a.q + b * a.qsb + h * a.qsh + s * a.qss + 8 * j));
-    const h8 xk = __builtin_nontemporal_load(reinterpret_cast<const h8 *>(a.k + b * a.ksb + h * a.ksh + s * a.kss + 8 * j));
+    const h8 *pxq = reinterpret_cast<const h8 *>(a.q + b * a.qsb + h * a.qsh + s * a.qss + 8 * j);
+    const h8 *pxk = reinterpret_cast<const h8 *>(a.k + b * a.ksb + h * a.ksh + s * a.kss + 8 * j);
+    const h8 xq = STREAM ? __builtin_nontemporal_load(pxq) : *pxq;
+    const h8 xk = STREAM ? __builtin_nontemporal_load(pxk) : *pxk;
     const h8 pq = swap4(xq), pk = swap4(xk);
     *reinterpret_cast<h8 *>(a.qo + b * a.oqb + h * a.oqh + s * a.oqs + 8 * j) = rope8(xq, pq, cs, snv, sg);
     *reinterpret_cast<h8 *>(a.ko + b * a.okb + h * a.okh + s * a.oks + 8 * j) = rope8(xk, pk, cs, snv, sg);
@@ -129,10 +127,15 @@ hipError_t launch_rope(const RopeArgs &a, bool backward, hipStream_t st) {
     if (vec) {
         const uint32_t rows = (uint32_t)a.B * (uint32_t)a.S * (uint32_t)a.H;
         const dim3 grid((rows + 31u) / 32u), block(256);
-        if (backward)
-            hipLaunchKernelGGL(rope_vec_kernel<true>, grid, block, 0, st, a);
+        const bool stream = rope_streams(a);
+        if (backward && stream)
+            hipLaunchKernelGGL((rope_vec_kernel<true, true>), grid, block, 0, st, a);
+        else if (backward)
+            hipLaunchKernelGGL((rope_vec_kernel<true, false>), grid, block, 0, st, a);
+        else if (stream)
+            hipLaunchKernelGGL((rope_vec_kernel<false, true>), grid, block, 0, st, a);
         else
-            hipLaunchKernelGGL(rope_vec_kernel<false>, grid, block, 0, st, a);
+            hipLaunchKernelGGL((rope_vec_kernel<false, false>), grid, block, 0, st, a);
     } else {
         const int nrb = (a.S + 7) / 8;
         const dim3 grid((unsigned)(nrb * a.B * a.H)), block(256);
