@@ -293,14 +293,14 @@ def test_fallback_calls_trace_and_take_nested_tensors():
     nested = torch.nested.nested_tensor(rows)
     jagged = torch.nested.nested_tensor([r.transpose(0, 1) for r in rows], layout=torch.jagged).transpose(1, 2)
     for t in (nested, jagged):
-        assert ready3(t, t, t) == -1 and ready3(q, q, t) == -1 and not fa.can_use(t, t, t)
+        assert ready3(t, t, t) == 16 and ready3(q, q, t) == 16 and not fa.can_use(t, t, t)
     assert not fa.can_use(q, None, None)   # an ineligible q settles it
     with FakeTensorMode():
         t = torch.empty(2, 3, 5, 64, device="cuda", dtype=torch.float16)
-        assert ready3(t, t, t) == -1 and fa.can_use(t, t, t) and not fa.can_use(t, t, t.float())
+        assert ready3(t, t, t) == 16 and fa.can_use(t, t, t) and not fa.can_use(t, t, t.float())
     seen = []
     make_fx(lambda x: seen.append((ready3(x, x, x), fa.can_use(x, x, x))) or x + 1, tracing_mode="symbolic")(q)
-    assert seen == [(-1, False)]
+    assert seen == [(16, False)]
 
 
 def test_eligibility_predicate_matches_reference_rules():

@@ -55,26 +55,30 @@ void strides3(const torch::Tensor &t, int64_t out[3]) {
 // The module's eligibility predicate (its _fa_ready: fp16 GPU (B,H,S,64), unit
 // stride in the head dimension, 32-byte aligned base and strides) of three
 // tensors in one call: bits 0..2 are q, k, v, bit 3 is set when all have one
-// shape; -1, and nothing asked of their sizes, if one is no plain strided
+// shape; 16, and nothing asked of their sizes, if one is no plain strided
 // tensor.  (From Python the three checks take 2.5 us, a quarter of a small
 // decode or prefill call's host time; here 0.4 us.)
-int64_t ready3(const torch::Tensor &q, const torch::Tensor &k, const torch::Tensor &v) {
-    const torch::Tensor *const ts[3] = {&q, &k, &v};
-    for (const torch::Tensor *t : ts) {
-        const c10::TensorImpl *impl = t->unsafeGetTensorImpl();
-        if (!t->defined() || t->layout() != c10::kStrided || t->is_nested() || impl->is_python_dispatch() ||
+int64_t ready3(pybind11::handle q, pybind11::handle k, pybind11::handle v) {
+    constexpr int64_t UNKNOWN = 16;
+    const pybind11::handle hs[3] = {q, k, v};
+    for (const pybind11::handle h : hs) {
+        if (!THPVariable_Check(h.ptr())) return UNKNOWN;
+        const torch::Tensor &t = THPVariable_Unpack(h.ptr());
+        const c10::TensorImpl *impl = t.unsafeGetTensorImpl();
+        if (t.layout() != c10::kStrided || t.is_nested() || impl->is_python_dispatch() ||
             impl->has_symbolic_sizes_strides())
-            return -1;
+            return UNKNOWN;
     }
     int64_t bits = 0;
     for (int i = 0; i < 3; ++i) {
-        const torch::Tensor &t = *ts[i];
+        const torch::Tensor &t = THPVariable_Unpack(hs[i].ptr());
         if (t.is_cuda() && t.scalar_type() == torch::kHalf && t.dim() == 4 && t.size(3) == 64 && t.stride(3) == 1 &&
             reinterpret_cast<uintptr_t>(t.data_ptr()) % 32 == 0 &&
             (t.stride(0) * 2) % 32 == 0 && (t.stride(1) * 2) % 32 == 0 && (t.stride(2) * 2) % 32 == 0)
             bits |= (int64_t)1 << i;
     }
-    if (q.sizes() == k.sizes() && q.sizes() == v.sizes()) bits |= 8;
+    const c10::IntArrayRef sizes = THPVariable_Unpack(q.ptr()).sizes();
+    if (sizes == THPVariable_Unpack(k.ptr()).sizes() && sizes == THPVariable_Unpack(v.ptr()).sizes()) bits |= 8;
     return bits;
 }
 

@@ -45,6 +45,7 @@ import os
 
 import torch
 import torch.nn.functional as F
+from torch.compiler import is_compiling
 
 _THIS_DIR = os.path.dirname(os.path.abspath(__file__))
 _LIB_DIR = os.path.join(_THIS_DIR, "lib")
@@ -176,31 +177,29 @@ def _fa_ready(t):
             and all((s * 2) % 32 == 0 for s in t.stride()[:3]))
 
 
-def _native_bits(q, k, v):
-    """_fa_ready of q, k, v in bits 0..2 and, in bit 3, whether their shapes agree, from one native
-    call; -1 where only _fa_ready can say: tensors that are not plain ones (nested, fake, symbolic
-    sizes, subclasses), a q on the CPU, and code under torch.compile, which cannot trace the call."""
-    if _EXT is None or not q.is_cuda or torch.compiler.is_compiling():
-        return -1
-    return _EXT.ready3(q, k, v)
+_UNKNOWN = 16
 
 
 def _ready_bits(q, k, v):
-    """_fa_ready of q, k, v in bits 0..2."""
-    bits = _native_bits(q, k, v)
-    return bits if bits >= 0 else _fa_ready(q) | _fa_ready(k) << 1 | _fa_ready(v) << 2
+    """_fa_ready of q, k, v in bits 0..2 and, in bit 3, whether their shapes agree, from one native
+    call; _UNKNOWN where only _fa_ready can say: tensors that are not plain ones (nested, fake,
+    symbolic sizes, subclasses) and code under torch.compile, which cannot trace the call."""
+    if _EXT is None or is_compiling():
+        return _UNKNOWN
+    return _EXT.ready3(q, k, v)
 
 
-def _all_ready(q, k, v):
-    bits = _native_bits(q, k, v)
-    return bits & 7 == 7 if bits >= 0 else _fa_ready(q) and _fa_ready(k) and _fa_ready(v)
+def _made_ready(ready, q, k, v):
+    """q, k, v with those that are not ready (_ready_bits) copied."""
+    return (t if ready >> i & 1 or (ready == _UNKNOWN and _fa_ready(t)) else t.contiguous()
+            for i, t in enumerate((q, k, v)))
 
 
 def can_use(q, k, v):
     """Whether the tensors can go to the kernel directly (reference :105-108)."""
-    bits = _native_bits(q, k, v)
-    if bits >= 0:
-        return bits == 15
+    ready = _ready_bits(q, k, v)
+    if ready != _UNKNOWN:
+        return ready == 15
     return (_fa_ready(q) and _fa_ready(k) and _fa_ready(v)
             and q.shape == k.shape == v.shape)
 
@@ -253,7 +252,7 @@ def flash_attn_v100(q, k, v, dropout_p: float = 0.0, causal: bool = True, softma
         raise ValueError("flash_attn_v100 only supports fp16 GPU tensors with head_dim=64")
     ready = _ready_bits(q, k, v)
     if ready & 7 != 7:
-        q, k, v = (t if ready >> i & 1 else t.contiguous() for i, t in enumerate((q, k, v)))
+        q, k, v = _made_ready(ready, q, k, v)
     if softmax_scale is None:
         softmax_scale = q.shape[-1] ** -0.5
     return _FlashAttnV100Cuda.apply(q, k, v, float(dropout_p), bool(causal), float(softmax_scale))
@@ -269,8 +268,9 @@ def _needs_grad(*ts):
 
 def _kv_ready(q, k, v):
     """fp16 (B,H,S_q,64) queries against (B,H,S_k,64) keys/values, kernel-aligned."""
-    return (_all_ready(q, k, v) and k.shape == v.shape
-            and k.shape[:2] == q.shape[:2] and k.size(2) >= 1)
+    ready = _ready_bits(q, k, v)
+    return ((ready & 7 == 7 if ready != _UNKNOWN else _fa_ready(q) and _fa_ready(k) and _fa_ready(v))
+            and k.shape == v.shape and k.shape[:2] == q.shape[:2] and k.size(2) >= 1)
 
 
 def _fwd_kv(q, k, v, causal, softmax_scale, causal_offset):
@@ -280,7 +280,7 @@ def _fwd_kv(q, k, v, causal, softmax_scale, causal_offset):
         raise RuntimeError("the key/value-length forward is inference-only (no backward)")
     ready = _ready_bits(q, k, v)
     if ready & 7 != 7:
-        q, k, v = (t if ready >> i & 1 else t.contiguous() for i, t in enumerate((q, k, v)))
+        q, k, v = _made_ready(ready, q, k, v)
     if softmax_scale is None:
         softmax_scale = 0.125   # 64 ** -0.5
     o, _ = extension().fa_fwd_kv(q, k, v, bool(causal), float(softmax_scale), int(causal_offset))
