@@ -942,7 +942,8 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdArgs a) {
 // V from HBM once; an MFMA tile would use one of its 32 query rows.
 // ---------------------------------------------------------------------------
 // Workgroup (slice ks, b*H + h) takes the keys of slice ks (all keys when
-// nsplit = 1) in 64-key blocks, wave w blocks w, w + DEC_NW, ...  Per block, lane L = 8g + c8 loads the 16-byte chunk c8 (dims 8*c8 .. +7) of key
+// nsplit = 1) in 64-key blocks, wave w blocks w, w + DEC_NW, ...  Per block,
+// lane L = 8g + c8 loads the 16-byte chunk c8 (dims 8*c8 .. +7) of key
 // rows k0 + 8i + g, i = 0..7, of K and of V (each of the eight loads covers 1 KB
 // of consecutive rows), forms the partial dot of its chunk with q's, and a
 // butterfly over the 8 lanes of group g gives all of them the score of row
