@@ -1213,8 +1213,8 @@ static hipError_t launch_decode(const FwdArgs &a_in, hipStream_t st) {
     const int64_t wgs = (int64_t)a.B * a.H * a.nsplit, per = 1 << 22;
     for (int64_t w = 0; w < wgs; w += per) {
         a.wg0 = (int)w;
-        hipLaunchKernelGGL((decode_kernel<CAUSAL, STREAM, DEC_NW>), dim3((unsigned)std::min(per, wgs - w)), dim3(DEC_NW * 64),
-                           0, st, a);
+        hipLaunchKernelGGL((decode_kernel<CAUSAL, STREAM, DEC_NW>), dim3((unsigned)std::min(per, wgs - w)),
+                           dim3(DEC_NW * 64), 0, st, a);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

@@ -182,10 +182,10 @@ int64_t auto_nsplit(int64_t wgs, int64_t tiles) {
 // 192 workgroups take 20.6 us, 288 take 24.8 and 96 take 24.9), slices of at
 // least 256 keys, and none below 1536 keys, where the merge's launch costs
 // more than the slices save (B*H = 12: S_k = 1000 5.8 us in one piece, 6.2 in
-// four, 6.7 in two; S_k = 2500 8.9 in one, 6.8 in nine).  From 80 heads on one workgroup a
-// head draws most of what the memory gives, and there are none below 2048 keys
-// (S_k = 1800: 80 heads 8.8 us in one piece, 9.4 in three; 128 heads 11.7 in
-// one, 14.1 in two).
+// four, 6.7 in two; S_k = 2500 8.9 in one, 6.8 in nine).  From 80 heads on one
+// workgroup a head draws most of what the memory gives, and there are none below
+// 2048 keys (S_k = 1800: 80 heads 8.8 us in one piece, 9.4 in three; 128 heads
+// 11.7 in one, 14.1 in two).
 int64_t auto_nsplit_decode(int64_t bh, int64_t s_k) {
     if (s_k < (bh < 80 ? 1536 : 2048)) return 1;
     int64_t n = (192 + bh - 1) / bh;
